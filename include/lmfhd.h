@@ -315,8 +315,9 @@ const char* lmfhd_last_error(void);
  * counterpart; its nearest knob is the tiling flag of mfiter_build (stag_applyop.f90:143-201). */
 typedef struct lmfhd_tune {
   int coarse_n;        /* staggered multigrid levels with every cell count <= coarse_n run as one
-                          one-workgroup kernel per V-cycle (0: none; at most 16) */
-  int mac_coarse_n;    /* the same for the MAC pressure multigrid */
+                          one-workgroup kernel per V-cycle (0: none; at most 16); from 8 on, so do
+                          larger levels that one workgroup can hold (about 12^3 in FP32, 9^3 in FP64) */
+  int mac_coarse_n;    /* the same for the MAC pressure multigrid (about 16^3 in FP32, 12^3 in FP64) */
   int coarse_threads;  /* threads of that workgroup: 256, 512 or 1024 */
   int red_blocks;      /* workgroups of an inner-product launch: 64 .. 4096 */
   int graphs;          /* 1: HIP-graph replay of Arnoldi steps (taken when lmfhd_desc.graphs = -1) */

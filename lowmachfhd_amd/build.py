@@ -6,7 +6,10 @@ import subprocess
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRC = os.path.join(HERE, "csrc", "lmfhd.hip")
+# translation units: (source, object, further flags); the coarse kernels once per precision
+UNITS = [(os.path.join(HERE, "csrc", src), os.path.join(HERE, "csrc", obj), extra) for src, obj, extra in (
+    ("lmfhd.hip", "lmfhd.o", []), ("coarse.hip", "coarse32.o", ["-DLMFHD_COARSE_T=float"]),
+    ("coarse.hip", "coarse64.o", ["-DLMFHD_COARSE_T=double"]))]
 OUT = os.path.join(HERE, "liblmfhd.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -17,19 +20,29 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # every launch form would not be; the kernels are memory-bound, so fused multiply-adds buy
 # nothing here.
 FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
 
 def build_library(verbose: bool = False) -> str:
-    cmd = [HIPCC, *FLAGS, "-o", OUT + ".tmp", SRC]
-    res = subprocess.run(cmd, capture_output=True, text=True)
+    """Compile the translation units side by side and link them."""
+    objs = [obj for _, obj, _ in UNITS]
+    procs = [subprocess.Popen([HIPCC, *FLAGS, *extra, "-c", "-o", obj, src], stdout=subprocess.PIPE,
+                              stderr=subprocess.STDOUT, text=True) for src, obj, extra in UNITS]
+    outs = [p.communicate()[0] for p in procs]
+    for (src, _, _), p, out in zip(UNITS, procs, outs):
+        if p.returncode != 0:
+            sys.stderr.write(out)
+            raise RuntimeError("hipcc failed for " + src)
+        if verbose:
+            sys.stderr.write(out)
+    res = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-o", OUT + ".tmp", *objs], capture_output=True, text=True)
+    for o in objs:
+        os.remove(o)
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed for " + SRC)
-    if verbose:
-        sys.stderr.write(res.stderr)
+        raise RuntimeError("linking failed for " + OUT)
     os.replace(OUT + ".tmp", OUT)
     return OUT
 

@@ -32,7 +32,7 @@ struct Rec {
   std::vector<unsigned char> f;   // the functor's bytes
   long n = 0;                     // flat: items; blocks: workgroups
   int ncols = 0, nz = 0, kc = 0;  // cols
-  int nw = 0;                     // rows: waves
+  int nw = 0;                     // rows: waves; blocks: threads of a workgroup
   MultiFn multi = nullptr;
 };
 struct Recorder {
@@ -254,8 +254,9 @@ void multi_rows(hipStream_t s, const unsigned char* fs, int nent, const Rec& r) 
 #endif
 }
 
-// Workgroup functors: F::block(b) runs workgroup b of a launch of nb workgroups of F::BS threads
-// (it may use __shared__ memory and barriers); launch_blocks runs them, recordable like the rest.
+// Workgroup functors: F::block(b) runs workgroup b of a launch of nb workgroups of F::BS threads, or
+// of fewer when the caller names a number (it may use __shared__ memory and barriers);
+// launch_blocks runs them, recordable like the rest.
 // In the host debug build a workgroup functor provides block_host(b) instead.
 #ifndef LMFHD_HOST_DEBUG
 template <class F>
@@ -274,23 +275,24 @@ void multi_blocks(hipStream_t s, const unsigned char* fs, int nent, const Rec& r
   for (int q = 0; q < nent; ++q)
     for (long b = 0; b < r.n; ++b) reinterpret_cast<const F*>(fs)[q].block_host((int)b);
 #else
-  hipLaunchKernelGGL(k_blocks_multi<F>, dim3((unsigned)r.n, (unsigned)nent), dim3(F::BS), 0, s,
+  hipLaunchKernelGGL(k_blocks_multi<F>, dim3((unsigned)r.n, (unsigned)nent), dim3((unsigned)r.nw), 0, s,
                      reinterpret_cast<const F*>(fs));
 #endif
 }
 template <class F>
-inline void launch_blocks(hipStream_t s, int nb, const F& f) {
+inline void launch_blocks(hipStream_t s, int nb, const F& f, int nt = F::BS) {
   static_assert(sizeof(F) + 32 <= MAX_KERNARG, "functor too large for the kernel-argument segment");
   if (nb <= 0) return;
   if (rec_slot()) {
-    record(3, f, &multi_blocks<F>, nb);
+    record(3, f, &multi_blocks<F>, nb, 0, 0, 0, nt);
     return;
   }
 #ifdef LMFHD_HOST_DEBUG
   (void)s;
+  (void)nt;
   for (int b = 0; b < nb; ++b) f.block_host(b);
 #else
-  hipLaunchKernelGGL(k_blocks<F>, dim3((unsigned)nb), dim3(F::BS), 0, s, f);
+  hipLaunchKernelGGL(k_blocks<F>, dim3((unsigned)nb), dim3((unsigned)nt), 0, s, f);
 #endif
 }
 

@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "../../include/lmfhd.h"
+#include "coarse.h"
 #include "launch.h"
 #include "stencils.h"
 
@@ -831,102 +832,6 @@ static bool even_level(const Geo& g) {
   return true;
 }
 
-// compile-time dispatch on (visc_type, dm)
-template <class F>
-static void dispatch_vd(int vt, int dm, F&& f) {
-#define LMFHD_VD(V, D) f(std::integral_constant<int, V>{}, std::integral_constant<int, D>{})
-  if (dm == 3) {
-    switch (vt) {
-      case -1: LMFHD_VD(-1, 3); break;
-      case -2: LMFHD_VD(-2, 3); break;
-      case -3: LMFHD_VD(-3, 3); break;
-      case 1: LMFHD_VD(1, 3); break;
-      case 2: LMFHD_VD(2, 3); break;
-      default: LMFHD_VD(3, 3); break;
-    }
-  } else {
-    switch (vt) {
-      case -1: LMFHD_VD(-1, 2); break;
-      case -2: LMFHD_VD(-2, 2); break;
-      case -3: LMFHD_VD(-3, 2); break;
-      case 1: LMFHD_VD(1, 2); break;
-      case 2: LMFHD_VD(2, 2); break;
-      default: LMFHD_VD(3, 2); break;
-    }
-  }
-#undef LMFHD_VD
-}
-
-
-// ------------------------------------------------------------------------------------------
-// Coarse levels in one workgroup.  Every level whose cell counts are all <= COARSE_N is
-// smoothed, restricted and prolongated by a single 1024-thread workgroup with a barrier
-// between phases, replacing ~10^2 tiny launches (each ~5 us of GPU time whatever its size) per
-// V-cycle by one.  Phase order and arithmetic are those of the per-level kernels.
-static const int COARSE_MAXL = 16;
-static const int COARSE_N = 16;
-static const int COARSE_THREADS = 1024;
-
-// LDS staging.  The arrays of the levels whose extents are all <= COARSE_N come from one block
-// per multigrid (the arena), coarsest level first, so the levels of a one-workgroup V-cycle
-// (level l0 and every coarser one) are one prefix of it.  When that prefix fits STAGE_BYTES
-// the kernel copies it into LDS, runs every phase on the LDS copies (a phase then waits on
-// LDS, not on L2, for its operands) and copies level l0's phi, the only result read later,
-// back.  The phases and their arithmetic are unchanged.
-static const unsigned STAGE_BYTES = 144u * 1024u;
-struct Arena {  // byte offsets of the small levels' arrays in the arena, 16-byte aligned
-  long bytes = 0;
-  long take(long nbytes) {
-    const long o = (bytes + 15) / 16 * 16;
-    bytes = o + nbytes;
-    return o;
-  }
-  long end() const { return (bytes + 15) / 16 * 16; }
-};
-struct StageInfo {
-  const unsigned char* arena;  // the arena in device memory
-  unsigned bytes;              // prefix staged in LDS (0: the V-cycle runs on device memory)
-  unsigned out_off, out_bytes; // level l0's phi within it
-};
-
-template <typename T>
-struct StagLevArgs {
-  Geo g;
-  T dxsqinv;
-  T* alpha[3];
-  T* beta;
-  T* gamma;
-  T* bed[3];
-  T* phi[3];
-  T* rhs[3];
-  T* res[3];
-  Dec dface[3], dcolor[3];  // decoders of the level's face arrays (all faces / one colour)
-};
-template <typename T>
-struct StagCoarseArgs {
-  int l0, nl, nu_down, nu_up, nu_bottom;
-  int fuse;  // one phase per parity for all components where they decouple (|visc_type| 1)
-  T omega;
-  StageInfo st;
-  StagLevArgs<T> L[COARSE_MAXL];
-};
-// The level table (several KB) exceeds the kernel-argument segment (launch.h), so it lives in
-// device memory, written by a completed copy from the host (h2d) before any kernel reads it.
-
-// The same per-component functor over the three components' item ranges in one phase
-// ([0, n0) component 0, [n0, n01) component 1, the rest component 2): for steps whose
-// components write disjoint arrays from inputs the phase does not change (residual,
-// restriction, prolongation).
-template <class F>
-struct Comp3Fn {
-  F f[3];
-  long n0, n01;
-  HD void operator()(long t) const {
-    if (t < n0) f[0](t);
-    else if (t < n01) f[1](t - n0);
-    else f[2](t - n01);
-  }
-};
 // The same functor over the components' item ranges in one flat launch, the components
 // alternating by workgroup (block b runs items 256 (b / DM) + [0, 256) of component b % DM): the
 // branch on the component is uniform in a workgroup
@@ -947,372 +852,32 @@ struct Comp3BlkFn {
     }
   }
 };
-template <class F, int DM, class Make, class Count>
-HD Comp3Fn<F> comp3(const Make& make, const Count& count, long& total) {
-  Comp3Fn<F> c{{make(0), make(DM > 1 ? 1 : 0), make(DM > 2 ? 2 : DM - 1)}, 0, 0};
-  const long c0 = count(0), c1 = DM > 1 ? count(1) : 0, c2 = DM > 2 ? count(2) : 0;
-  c.n0 = c0;
-  c.n01 = c0 + c1;
-  total = c0 + c1 + c2;
-  return c;
+// Levels a one-workgroup V-cycle takes (lmfhd_tune.coarse_n, mac_coarse_n = cn): those with every
+// extent <= cn and, from cn = 8 on, any level whose faces (cells) a workgroup of 1024 threads
+// holds in registers and whose work block fits LDS (|visc_type| 1: 3-D boxes up to about 12^3 in
+// FP32 and 9^3 in FP64, 2-D ones up to 48^2 and 32^2; MAC levels up to 16^3 in FP32, 12^3 in
+// FP64, 2-D 64^2).  slots_max: what a thread holds.
+static bool coarse_fits(const Geo& g, int cn, int slots, int slots_max, long work_bytes) {
+  bool small = true;
+  for (int d = 0; d < g.dm; ++d) if (g.n[d] > cn) small = false;
+  return small || (cn >= 8 && slots <= slots_max * COARSE_THREADS && work_bytes <= (long)COARSE_LDS);
 }
-template <typename T, int VT, int DM, class Run, class Map>
-HD void stag_coarse_body(const StagCoarseArgs<T>& A, Run& run, const Map& M) {
-  // phi of level l0 > 0 arrives zeroed (the restriction launch before this kernel), and each
-  // restriction below zeroes phi of the level it writes; level 0's phi (l0 = 0) is the initial
-  // guess
-  auto coefs = [&](int n) __attribute__((always_inline)) {
-    Coefs<T> C;
-    for (int d = 0; d < 3; ++d) { C.alpha[d] = M(A.L[n].alpha[d]); C.bed[d] = M(A.L[n].bed[d]); }
-    C.beta = M(A.L[n].beta);
-    C.gamma = M(A.L[n].gamma);
-    C.dxsqinv = A.L[n].dxsqinv;
-    C.theta = T(1);
-    return C;
-  };
-  auto smooth = [&](int n, int nsweeps) __attribute__((always_inline)) {
-    const StagLevArgs<T>& l = A.L[n];
-    const Coefs<T> C = coefs(n);
-    bool inplace = true;
-    for (int d = 0; d < DM; ++d) if (l.g.n[d] % 2) inplace = false;
-    for (int m = 0; m < nsweeps; ++m) {
-      if constexpr (VT == 1 || VT == -1) {
-        if (inplace && A.fuse) {  // one phase per parity for all components (GsColorAllFn)
-          GsColorAllFn<T, VT, DM> F;
-          F.g = l.g;
-          F.C = C;
-          long cum = 0, ncs[3] = {0, 0, 0};
-          for (int a = 0; a < DM; ++a) {
-            F.phi[a] = M(l.phi[a]);
-            F.rhs[a] = M(l.rhs[a]);
-            F.dc[a] = l.dcolor[a];
-            ncs[a] = (long)((fext(l.g, a, 0) + 1) / 2) * fext(l.g, a, 1) * fext(l.g, a, 2);
-          }
-          for (int a = DM; a < 3; ++a) { F.phi[a] = M(l.phi[DM - 1]); F.rhs[a] = M(l.rhs[DM - 1]); F.dc[a] = l.dcolor[DM - 1]; }
-          // each component's items from a wave boundary: a wave then holds one component and
-          // takes one branch of the component dispatch (on the smallest levels a wave would
-          // otherwise run the three components' stencils one after the other)
-          for (int a = 0; a < 3; ++a) F.nc[a] = a < DM ? (unsigned)ncs[a] : 0u;
-          F.n0 = (ncs[0] + 63) / 64 * 64;
-          F.n01 = F.n0 + (ncs[1] + 63) / 64 * 64;
-          F.ilv = 0;
-          cum = DM == 3 ? F.n01 + ncs[2] : F.n0 + ncs[1];
-          F.omega = A.omega;
-          for (int par = 0; par < 2; ++par) {
-            F.par = par;
-            run(F, cum);
-          }
-          continue;
-        }
-      }
-      for (int color = 1; color <= 2 * DM; ++color) {
-        const int a = (color - 1) / 2, par = (color + 1) % 2;
-        const int nx = fext(l.g, a, 0), ny = fext(l.g, a, 1);
-        const long nc = (long)((nx + 1) / 2) * ny * fext(l.g, a, 2);
-        if (inplace) {
-          run(GsColorFn<T, VT, DM>{l.g, C, {M(l.phi[0]), M(l.phi[1]), M(l.phi[2])}, M(l.rhs[a]), A.omega, a, l.dcolor[a], par}, nc);
-        } else {
-          run(ApplyColorFn<T, VT, DM>{l.g, C, {M(l.phi[0]), M(l.phi[1]), M(l.phi[2])}, M(l.res[a]), a, l.dcolor[a], par}, nc);
-          run(UpdateColorFn<T, VT, DM>{l.g, C, M(l.phi[a]), M(l.rhs[a]), M(l.res[a]), A.omega, a, l.dcolor[a], par}, nc);
-        }
-      }
-    }
-  };
-  for (int n = A.l0; n < A.nl - 1; ++n) {
-    smooth(n, A.nu_down);
-    const StagLevArgs<T>& f = A.L[n];
-    const StagLevArgs<T>& c = A.L[n + 1];
-    const Coefs<T> C = coefs(n);
-    long cnt = 0;
-    const auto R = comp3<ApplyFn<T, VT, DM>, DM>(
-        [&](int a) { return ApplyFn<T, VT, DM>{f.g, C, {M(f.phi[0]), M(f.phi[1]), M(f.phi[2])}, M(f.rhs[a]), M(f.res[a]), a, f.dface[a], 1}; },
-        [&](int a) { return fsize(f.g, a); }, cnt);
-    run(R, cnt);
-    const auto Q = comp3<RestrictFn<T, DM>, DM>(
-        [&](int a) { return RestrictFn<T, DM>{f.g, c.g, M(f.res[a]), M(c.rhs[a]), a, c.dface[a], 0, 0, 0, M(c.phi[a])}; },
-        [&](int a) { return fsize(c.g, a); }, cnt);
-    run(Q, cnt);
-  }
-  smooth(A.nl - 1, A.nu_bottom);
-  for (int n = A.nl - 2; n >= A.l0; --n) {
-    const StagLevArgs<T>& f = A.L[n];
-    const StagLevArgs<T>& c = A.L[n + 1];
-    long cnt = 0;
-    const auto P = comp3<ProlongFn<T, DM>, DM>(
-        [&](int a) { return ProlongFn<T, DM>{f.g, c.g, M(f.phi[a]), M(c.phi[a]), a, f.dface[a]}; },
-        [&](int a) { return fsize(f.g, a); }, cnt);
-    run(P, cnt);
-    smooth(n, A.nu_up);
-  }
-}
-
-template <typename T>
-struct MacLevArgs {
-  Geo g;
-  T h2i;
-  T* b[3];
-  T* phi;
-  T* rhs;
-  T* tmp;
-  Dec dcell, dcolor;
-};
-template <typename T>
-struct MacCoarseArgs {
-  int l0, nl, nu_down, nu_up, nu_bottom;
-  StageInfo st;
-  MacLevArgs<T> L[COARSE_MAXL];
-};
-
-// the LDS staging of a coarse V-cycle from level l0 (StageInfo): the arena prefix of levels
-// l0 .. nl-1 when it fits STAGE_BYTES; level l0's phi block goes back.  LMFHD_STAGE=0 when the
-// context is built turns it off (the V-cycle then runs on device memory, with the same bits)
-static StageInfo stage_info(const unsigned char* arena, int arena_l, const std::vector<long>& lev_end,
-                            long phi_off, long phi_bytes, int l0) {
+// The kernel for a coarse V-cycle whose first level has so many slots (coarser ones have fewer).
+// LMFHD_STAGE=0 when the context is built runs it on device memory (same bits)
+static CoarseForm coarse_kernel_form(long work_bytes, int slots, int nt) {
   const char* e = getenv("LMFHD_STAGE");
-  const bool off = e && e[0] == '0';
-  StageInfo st{arena, 0u, 0u, 0u};
-  if (off || !arena || l0 < arena_l || l0 >= (int)lev_end.size() || lev_end[l0] > (long)STAGE_BYTES) return st;
-  st.bytes = (unsigned)lev_end[l0];
-  st.out_off = (unsigned)phi_off;
-  st.out_bytes = (unsigned)phi_bytes;
-  return st;
-}
-
-// The coarse bodies take every array through a map: the identity on device memory; for a
-// staged V-cycle, an arena address to the same offset in the LDS block (formed from the block
-// itself, so the compiler addresses LDS directly: 32-bit offsets and LDS instructions)
-struct NoMap {
-  template <typename P>
-  HD P operator()(P p) const { return p; }
-};
-struct StageMap {
-  const unsigned char* arena;
-  unsigned char* buf;
-  template <typename P>
-  HD P operator()(P p) const { return (P)(buf + (unsigned)((const unsigned char*)p - arena)); }
-};
-
-template <typename T, int DM, class Run, class Mean, class Map>
-HD void mac_coarse_body(const MacCoarseArgs<T>& A, Run& run, Mean& remove_mean, const Map& M) {
-  // phi of level l0 > 0 arrives zeroed, and each restriction below zeroes the level it writes
-  auto gs = [&](int n, int nsweeps) __attribute__((always_inline)) {
-    const MacLevArgs<T>& l = A.L[n];
-    bool inplace = true;
-    for (int d = 0; d < DM; ++d) if (l.g.n[d] % 2) inplace = false;
-    const long nc = (long)((l.g.n[0] + 1) / 2) * l.g.n[1] * l.g.n[2];
-    for (int m = 0; m < nsweeps; ++m)
-      for (int par = 0; par < 2; ++par) {
-        if (inplace) {
-          run(MacGsFn<T, DM>{l.g, {M(l.b[0]), M(l.b[1]), M(l.b[2])}, l.h2i, M(l.phi), M(l.rhs), par, l.dcolor}, nc);
-        } else {
-          run(MacGsNewFn<T, DM>{l.g, {M(l.b[0]), M(l.b[1]), M(l.b[2])}, l.h2i, M(l.phi), M(l.rhs), M(l.tmp), par, l.dcolor}, nc);
-          run(CopyColorCellFn<T>{l.g, M(l.phi), M(l.tmp), par, l.dcolor}, nc);
-        }
-      }
-  };
-  for (int n = A.l0; n < A.nl - 1; ++n) {
-    gs(n, A.nu_down);
-    const MacLevArgs<T>& f = A.L[n];
-    const MacLevArgs<T>& c = A.L[n + 1];
-    run(MacResidRestrictFn<T, DM>{f.g, c.g, {M(f.b[0]), M(f.b[1]), M(f.b[2])}, f.h2i, M(f.phi), M(f.rhs), M(c.rhs), c.dcell, M(c.phi)}, csize(c.g));
-  }
-  remove_mean(M(A.L[A.nl - 1].rhs), csize(A.L[A.nl - 1].g));
-  gs(A.nl - 1, A.nu_bottom);
-  for (int n = A.nl - 2; n >= A.l0; --n) {
-    run(MacProlongFn<T>{A.L[n].g, A.L[n + 1].g, M(A.L[n].phi), M(A.L[n + 1].phi), A.L[n].dcell}, csize(A.L[n].g));
-    gs(n, A.nu_up);
-  }
-}
-
-#ifndef LMFHD_HOST_DEBUG
-struct BlockRun {
-  template <class F>
-  __device__ __forceinline__ void operator()(const F& f, long n) const {
-    for (long t = threadIdx.x; t < n; t += blockDim.x) f(t);
-    __syncthreads();
-  }
-  // each component's items as a loop of its own: choosing the functor per lane made the
-  // compiler index the functor array with a lane-varying offset, which kept it in scratch
-  // Component a's loop starts a ring of a third of the workgroup's waves further on, so that on
-  // the small levels, where each component has fewer items than threads, the three run on
-  // different waves at once instead of one after the other (the items of a phase are
-  // independent, so which thread takes which does not change the result)
-  template <class F>
-  __device__ __forceinline__ void operator()(const Comp3Fn<F>& c, long n) const {
-    const long n1 = c.n01 - c.n0, n2 = n - c.n01;
-    const unsigned nt = blockDim.x, sh = ((nt >> 6) / 3) * 64;  // 2 sh < nt
-    const long t1 = (threadIdx.x + nt - sh) % nt, t2 = (threadIdx.x + nt - 2 * sh) % nt;
-    for (long t = threadIdx.x; t < c.n0; t += nt) c.f[0](t);
-    for (long t = t1; t < n1; t += nt) c.f[1](t);
-    for (long t = t2; t < n2; t += nt) c.f[2](t);
-    __syncthreads();
-  }
-};
-
-
-template <typename T>
-struct BlockMean {  // subtract the mean of x[0, n) (workgroup reduction in FP64)
-  __device__ void operator()(T* x, long n) const {
-    __shared__ double sh[COARSE_THREADS / 64];
-    double s = 0.0;
-    for (long e = threadIdx.x; e < n; e += blockDim.x) s += (double)x[e];
-    s = wave_sum(s);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    double tot = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) tot += sh[w];
-    const double mean = tot / (double)n;
-    __syncthreads();
-    for (long e = threadIdx.x; e < n; e += blockDim.x) x[e] = T((double)x[e] - mean);
-    __syncthreads();
-  }
-};
-
-// bytes (a multiple of 4) from src to dst by the workgroup: 16-byte words (both ends are
-// 16-byte aligned: arena offsets and the LDS block), up to 8 loads of a thread in flight (past
-// the end they reread the last word, and are not stored), then the 4-byte tail.  A native
-// vector type: the HIP uint4 struct kept the staging array in scratch
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void blk_copy(void* dst, const void* src, unsigned bytes) {
-  const unsigned n16 = bytes / 16, nt = blockDim.x, tid = threadIdx.x;
-  const u32x4* s4 = (const u32x4*)src;
-  u32x4* d4 = (u32x4*)dst;
-  for (unsigned b = 0; b < n16; b += 8 * nt) {
-    u32x4 v[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const unsigned e = b + k * nt + tid;
-      v[k] = s4[e < n16 ? e : n16 - 1];
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const unsigned e = b + k * nt + tid;
-      if (e < n16) d4[e] = v[k];
-    }
-  }
-  const unsigned* s1 = (const unsigned*)src;
-  unsigned* d1 = (unsigned*)dst;
-  for (unsigned e = n16 * 4 + tid; e < bytes / 4; e += nt) d1[e] = s1[e];
-}
-// a coarse V-cycle on LDS copies of its levels (StageInfo): arena prefix in, body through
-// StageMap, level l0's phi out
-template <class Args, class Body>
-__device__ __forceinline__ void staged_block(const Args& A, const Body& body) {
-  __shared__ __align__(16) unsigned char buf[STAGE_BYTES];
-  blk_copy(buf, A.st.arena, A.st.bytes);
-  __syncthreads();
-  body(StageMap{A.st.arena, buf});
-  __syncthreads();
-  blk_copy((void*)(A.st.arena + A.st.out_off), buf + A.st.out_off, A.st.out_bytes);
-}
-
-#else
-struct HostRun {
-  template <class F>
-  void operator()(const F& f, long n) const {
-    for (long t = 0; t < n; ++t) f(t);
-  }
-};
-template <typename T>
-struct HostMean {
-  void operator()(T* x, long n) const {
-    double acc = 0.0;
-    for (long e = 0; e < n; ++e) acc += (double)x[e];
-    const double m = acc / (double)n;
-    for (long e = 0; e < n; ++e) x[e] = T((double)x[e] - m);
-  }
-};
-// the LDS staging of staged_block with a host buffer in place of LDS (checks the arena layout
-// and the pointer map in a CPU build)
-template <class Args, class Body>
-void staged_block_host(const Args& A, const Body& body) {
-  std::vector<unsigned char> buf(STAGE_BYTES);
-  memcpy(buf.data(), A.st.arena, A.st.bytes);
-  body(StageMap{A.st.arena, buf.data()});
-  memcpy((void*)(A.st.arena + A.st.out_off), buf.data() + A.st.out_off, A.st.out_bytes);
-}
-
-#endif
-
-// The coarse V-cycle kernels as workgroup functors (launch_blocks, recordable): one workgroup
-// of NT threads runs the body on its argument block.  NT threads: 1024 caps a thread at 128
-// VGPRs (the stencils then spill to scratch); 256 and 512 leave room at the price of fewer
-// lanes per colour step.
-template <typename T, int VT, int DM, int NT>
-struct StagCoarseBlk {
-  static constexpr int BS = NT;
-  const StagCoarseArgs<T>* A;
-#ifdef LMFHD_HOST_DEBUG
-  void block_host(int) const {
-    const StagCoarseArgs<T>& a = *A;
-    auto body = [&](const auto& M) {
-      HostRun run;
-      stag_coarse_body<T, VT, DM>(a, run, M);
-    };
-    if (a.st.bytes) staged_block_host(a, body);
-    else body(NoMap{});
-  }
-#else
-  // inlined into the kernel: as a called function the body kept the callee-saved registers of
-  // the calling convention in scratch and spilled (248 VGPRs, 840 B of scratch per lane)
-  __device__ __forceinline__ void block(int) const {
-    const StagCoarseArgs<T>& a = *A;
-    auto body = [&](const auto& M) __attribute__((always_inline)) {
-      BlockRun run;
-      stag_coarse_body<T, VT, DM>(a, run, M);
-    };
-    if (a.st.bytes) staged_block(a, body);
-    else body(NoMap{});
-  }
-#endif
-};
-template <typename T, int DM, int NT>
-struct MacCoarseBlk {
-  static constexpr int BS = NT;
-  const MacCoarseArgs<T>* A;
-#ifdef LMFHD_HOST_DEBUG
-  void block_host(int) const {
-    const MacCoarseArgs<T>& a = *A;
-    auto body = [&](const auto& M) {
-      HostRun run;
-      HostMean<T> mean;
-      mac_coarse_body<T, DM>(a, run, mean, M);
-    };
-    if (a.st.bytes) staged_block_host(a, body);
-    else body(NoMap{});
-  }
-#else
-  __device__ __forceinline__ void block(int) const {
-    const MacCoarseArgs<T>& a = *A;
-    auto body = [&](const auto& M) __attribute__((always_inline)) {
-      BlockRun run;
-      BlockMean<T> mean;
-      mac_coarse_body<T, DM>(a, run, mean, M);
-    };
-    if (a.st.bytes) staged_block(a, body);
-    else body(NoMap{});
-  }
-#endif
-};
-
-static int coarse_level(const Geo& g0, int nl, int cn) {  // first level with all n_d <= cn
-  Geo g = g0;
-  for (int n = 0; n < nl; ++n) {
-    bool small = true;
-    for (int d = 0; d < g.dm; ++d) if (g.n[d] > cn) small = false;
-    if (small) return (nl <= COARSE_MAXL) ? n : nl;
-    g = coarsen_geo(g);
-  }
-  return nl;
+  if ((e && e[0] == '0') || work_bytes > (long)COARSE_LDS) return CoarseForm::device;
+  return slots <= SLOTS_SMALL * nt ? CoarseForm::lds_small : CoarseForm::lds;
 }
 
 // ------------------------------------------------------------------------------------------
 // colour launches of at least this many items interleave the components by workgroup
 constexpr long GS_ILV_MIN = 1L << 16;
-// levels whose every extent is at least this store phi, rhs, residual and alpha split by
-// parity (|visc_type| 1 with the Gauss-Seidel smoother on even sizes; far above the coarse
-// kernel's levels, which stay in natural storage)
+// levels whose every extent is at least this, of at least so many cells, store phi, rhs, residual
+// and alpha split by parity (|visc_type| 1 with the Gauss-Seidel smoother on even sizes; above
+// the coarse kernel's levels, which stay in natural storage)
 constexpr int SPLIT_MIN_N = 32;
+constexpr long SPLIT_MIN_CELLS = 4096;
 
 // Staggered velocity multigrid for (theta alpha - A0) phi = rhs in precision T.
 
@@ -1373,64 +938,72 @@ struct StagMG {
       g = coarsen_geo(g);
       h *= 2.0;
     }
-    // the small levels' arrays in the arena, coarsest level first (the coarse kernel's LDS
-    // staging); the rest in allocations of their own.  Everything starts zeroed (split storage
-    // has slack slots, odd extents, that are never written)
-    arena_l = nl;
-    while (arena_l > 0) {
-      bool small = true;
-      for (int d = 0; d < dm; ++d) if (L[arena_l - 1].g.n[d] > COARSE_N) small = false;
-      if (!small) break;
-      --arena_l;
+    // phi, rhs and res of the small levels in one work block, coarsest level first: the levels of
+    // a coarse V-cycle are a prefix of it, which the kernel holds in LDS.  The rest in
+    // allocations of their own.  Everything starts zeroed (split storage has slack slots, odd
+    // extents, that are never written)
+    work_l = nl;
+    work_off.assign(nl, 0);
+    long end = 0;
+    while (work_l > 0) {
+      const Geo& gl = L[work_l - 1].g;
+      const long o = end + 3 * stag_span(gl);
+      if (o > COARSE_WORK_MAX || L[work_l - 1].sp) break;
+      --work_l;
+      work_off[work_l] = end;
+      end = o;
     }
-    Arena ar;
-    lev_end.assign(nl, 0);
-    std::vector<std::array<long, 17>> offs(nl);
-    for (int n = nl - 1; n >= arena_l; --n) {
+    work = work_l < nl ? mem.alloc_zero<T>(end) : nullptr;
+    // their coefficients in one block too (fewer allocations)
+    const int nedge = dm == 3 ? 3 : 1;
+    auto pad = [](long n) { return (n + 63) / 64 * 64; };
+    long ncoef = 0;
+    for (int n = work_l; n < nl; ++n) {
       const Geo& gl = L[n].g;
-      auto& o = offs[n];
-      for (int a = 0; a < dm; ++a) o[a] = ar.take(fstore(gl, a, 0) * (long)sizeof(T));
-      o[3] = ar.take(csize(gl) * (long)sizeof(T));
-      o[4] = ar.take(csize(gl) * (long)sizeof(T));
-      for (int e = 0; e < (dm == 3 ? 3 : 1); ++e) o[5 + e] = ar.take(esize(gl, e) * (long)sizeof(T));
-      o[8] = ar.take(L[n].phi_span * (long)sizeof(T));
-      for (int a = 0; a < dm; ++a) o[11 + a] = ar.take(fstore(gl, a, 0) * (long)sizeof(T));
-      for (int a = 0; a < dm; ++a) o[14 + a] = ar.take(fstore(gl, a, 0) * (long)sizeof(T));
-      lev_end[n] = ar.end();
+      ncoef += stag_span(gl) + 2 * pad(csize(gl));
+      for (int e = 0; e < nedge; ++e) ncoef += pad(esize(gl, e));
     }
-    arena = arena_l < nl ? mem.alloc_zero<unsigned char>(ar.end()) : nullptr;
-    phi_off_l.assign(nl, 0);
+    T* cnext = work_l < nl ? mem.alloc_zero<T>(ncoef) : nullptr;
     for (int n = 0; n < nl; ++n) {
       Lev& l = L[n];
       const Geo& gl = l.g;
-      const bool in_arena = n >= arena_l;
-      auto get = [&](int slot, long count) {
-        return in_arena ? (T*)(arena + offs[n][slot]) : mem.alloc_zero<T>(count);
+      const bool in_work = n >= work_l;
+      auto coef = [&](long count) {
+        if (!in_work) return mem.alloc_zero<T>(count);
+        T* p = cnext;
+        cnext += pad(count);
+        return p;
       };
-      T* phis = get(8, l.phi_span);
-      phi_off_l[n] = in_arena ? offs[n][8] : 0;
+      T* phis = in_work ? work + work_off[n] : mem.alloc_zero<T>(l.phi_span);
       long off = 0;
       for (int a = 0; a < dm; ++a) {
         const long ns = fstore(gl, a, l.sp);
-        l.alpha[a] = get(a, ns);
+        l.alpha[a] = coef(ns);
         l.phi[a] = phis + off;
-        off += (ns + 63) / 64 * 64;
-        l.rhs[a] = get(11 + a, ns);
-        l.res[a] = get(14 + a, ns);
+        l.rhs[a] = in_work ? l.phi[a] + l.phi_span : mem.alloc_zero<T>(ns);
+        l.res[a] = in_work ? l.phi[a] + 2 * l.phi_span : mem.alloc_zero<T>(ns);
+        off += pad(ns);
       }
-      l.beta = get(3, csize(gl));
-      l.gamma = get(4, csize(gl));
-      for (int e = 0; e < (dm == 3 ? 3 : 1); ++e) l.bed[e] = get(5 + e, esize(gl, e));
+      l.beta = coef(csize(gl));
+      l.gamma = coef(csize(gl));
+      for (int e = 0; e < nedge; ++e) l.bed[e] = coef(esize(gl, e));
     }
   }
-  // the arena: levels arena_l .. nl-1; lev_end[n] = end of level n's part (levels n .. nl-1 are
-  // its prefix); phi_off_l[n] = offset of level n's phi block
-  unsigned char* arena = nullptr;
-  int arena_l = 0;
-  std::vector<long> lev_end, phi_off_l;
+  T* work = nullptr;  // levels work_l .. nl-1; level n's three blocks start at element work_off[n]
+  int work_l = 0;
+  std::vector<long> work_off;
+  // the first level a coarse V-cycle may start at under lmfhd_tune.coarse_n = cn (nl: none)
+  int coarse_start(int cn) const {
+    int l0 = nl;
+    while (l0 > std::max(work_l, nl - COARSE_MAXL) &&
+           coarse_fits(L[l0 - 1].g, cn, stag_slots(L[l0 - 1].g, vt, nullptr), stag_slots_max<T>(vt),
+                       (work_off[l0 - 1] + 3 * L[l0 - 1].phi_span) * (long)sizeof(T)))
+      --l0;
+    return l0;
+  }
 
   bool split_level(const Geo& g) const {
-    if (smoother != 1 || (vt != 1 && vt != -1) || !even_level(g)) return false;
+    if (smoother != 1 || (vt != 1 && vt != -1) || !even_level(g) || csize(g) < SPLIT_MIN_CELLS) return false;
     for (int d = 0; d < dm; ++d)
       if (g.n[d] < SPLIT_MIN_N) return false;
     return true;
@@ -1676,57 +1249,65 @@ struct StagMG {
     launch(s, (long)DM * ((mx + 255) / 256) * 256, F);
   }
 
-  // levels l0..nl-1 of one V-cycle in one workgroup (phi of levels >= max(l0,1) zeroed by the
-  // restrictions into them); the argument block (pointers and decoders of every level) lives in
-  // device memory
+  // levels l0..nl-1 of one V-cycle in one workgroup (coarse.h); phi of level l0 > 0 arrives zeroed
+  // by the restriction into it.  The argument block (offsets and decoders of every level) lives
+  // in device memory
   StagCoarseArgs<T>* coarse_args = nullptr;
   int coarse_l0 = -1;
-  int coarse_nt = 512;  // threads of the one-workgroup kernel: 256, 512 or 1024
-  void build_coarse(int l0, int nt, hipStream_t s, DevMem& mem) {
+  int coarse_nt = COARSE_THREADS;
+  CoarseForm coarse_form = CoarseForm::lds;
+  void build_coarse(int cn, int nt, hipStream_t s, DevMem& mem) {
+    const int l0 = coarse_start(cn);
     coarse_l0 = l0;
     coarse_nt = nt;
     if (l0 >= nl) return;
-    StagCoarseArgs<T> A;
-    memset(&A, 0, sizeof(A));
-    A.l0 = l0;
-    A.nl = nl;
+    std::unique_ptr<StagCoarseArgs<T>> Ap(new StagCoarseArgs<T>);
+    StagCoarseArgs<T>& A = *Ap;
+    memset((void*)&A, 0, sizeof(A));
+    A.l0 = 0;  // the table holds levels l0 .. nl-1
+    A.nl = nl - l0;
     A.nu_down = nu_down;
     A.nu_up = nu_up;
     A.nu_bottom = nu_bottom;
     A.omega = omega;
-    A.fuse = 1;
+    A.work = work;
+    coarse_form = coarse_kernel_form((work_off[l0] + 3 * L[l0].phi_span) * (long)sizeof(T), stag_slots(L[l0].g, vt, nullptr), nt);
     for (int n = l0; n < nl; ++n) {
-      StagLevArgs<T>& a = A.L[n];
+      StagLevArgs<T>& a = A.L[n - l0];
       const Lev& l = L[n];
       a.g = l.g;
       a.dxsqinv = l.dxsqinv;
-      for (int d = 0; d < 3; ++d) {
+      a.inplace = even_level(l.g);
+      stag_slots(l.g, vt, a.start);
+      a.phi = (int)work_off[n];
+      a.span = (int)l.phi_span;
+      int fs = 0;
+      for (int d = 0; d < dm; ++d) {
+        a.nx[d] = fext(l.g, d, 0);
+        a.nxy[d] = a.nx[d] * fext(l.g, d, 1);
+        a.nc[d] = (a.nx[d] + 1) / 2 * fext(l.g, d, 1) * fext(l.g, d, 2);
+        a.off[d] = (int)(l.phi[d] - l.phi[0]);
+        a.fstart[d] = fs;
+        a.nf[d] = (int)fsize(l.g, d);
+        fs += pad64(a.nf[d]);
+        a.dface[d] = make_dec(fext(l.g, d, 0), fext(l.g, d, 1));
+        a.dcolor[d] = make_dec_color(fext(l.g, d, 0), fext(l.g, d, 1));
         a.alpha[d] = l.alpha[d];
-        a.bed[d] = l.bed[d];
-        a.phi[d] = l.phi[d];
-        a.rhs[d] = l.rhs[d];
-        a.res[d] = l.res[d];
-        if (d < dm) {
-          a.dface[d] = make_dec(fext(l.g, d, 0), fext(l.g, d, 1));
-          a.dcolor[d] = make_dec_color(fext(l.g, d, 0), fext(l.g, d, 1));
-        }
+      }
+      a.fstart[dm] = fs;
+      for (int e = 0; e < (dm == 3 ? 3 : 1); ++e) {
+        a.enx[e] = eext(l.g, e, 0);
+        a.enxy[e] = a.enx[e] * eext(l.g, e, 1);
+        a.bed[e] = l.bed[e];
       }
       a.beta = l.beta;
       a.gamma = l.gamma;
     }
-    A.st = stage_info(arena, arena_l, lev_end, phi_off_l[l0], L[l0].phi_span * (long)sizeof(T), l0);
     if (!coarse_args) coarse_args = mem.alloc<StagCoarseArgs<T>>(1);
     h2d(coarse_args, &A, sizeof(A), s);
   }
-  void coarse(hipStream_t s, int l0) {
-    (void)l0;
-    dispatch_vd(vt, dm, [&](auto V, auto D) {
-      constexpr int VT = decltype(V)::value, DM = decltype(D)::value;
-      const int nt = coarse_nt;
-      if (nt == 256) launch_blocks(s, 1, StagCoarseBlk<T, VT, DM, 256>{coarse_args});
-      else if (nt == 512) launch_blocks(s, 1, StagCoarseBlk<T, VT, DM, 512>{coarse_args});
-      else launch_blocks(s, 1, StagCoarseBlk<T, VT, DM, 1024>{coarse_args});
-    });
+  void coarse(hipStream_t s) {
+    launch_stag_coarse<T>(s, vt, dm, coarse_nt, coarse_form, coarse_args);
     check_launch();
   }
 
@@ -1758,7 +1339,7 @@ struct StagMG {
         restrict_res(s, n);
       }
       if (l0 < nl) {
-        coarse(s, l0);
+        coarse(s);
       } else {
         smooth(s, nl - 1, nu_bottom);
       }
@@ -1812,39 +1393,44 @@ struct MacMG {
       g = coarsen_geo(g);
       h *= 2.0;
     }
-    // the small levels in the arena, coarsest first (the coarse kernel's LDS staging)
-    arena_l = nl;
-    while (arena_l > 0) {
-      bool small = true;
-      for (int d = 0; d < dm; ++d) if (L[arena_l - 1].g.n[d] > COARSE_N) small = false;
-      if (!small) break;
-      --arena_l;
+    // phi, rhs and residual of the small levels in one work block, as in StagMG
+    work_l = nl;
+    work_off.assign(nl, 0);
+    long end = 0;
+    while (work_l > 0) {
+      const long o = end + 3 * mac_span(L[work_l - 1].g);
+      if (o > COARSE_WORK_MAX) break;
+      --work_l;
+      work_off[work_l] = end;
+      end = o;
     }
-    Arena ar;
-    lev_end.assign(nl, 0);
-    std::vector<std::array<long, 6>> offs(nl);
-    for (int n = nl - 1; n >= arena_l; --n) {
-      const Geo& gl = L[n].g;
-      for (int a = 0; a < dm; ++a) offs[n][a] = ar.take(fsize(gl, a) * (long)sizeof(T));
-      for (int q = 3; q < 6; ++q) offs[n][q] = ar.take(csize(gl) * (long)sizeof(T));
-      lev_end[n] = ar.end();
-    }
-    arena = arena_l < nl ? mem.alloc_zero<unsigned char>(ar.end()) : nullptr;
-    phi_off_l.assign(nl, 0);
+    work = work_l < nl ? mem.alloc_zero<T>(end) : nullptr;
+    long ncoef = 0;
+    for (int n = work_l; n < nl; ++n) ncoef += stag_span(L[n].g);
+    T* cnext = work_l < nl ? mem.alloc<T>(ncoef) : nullptr;
     for (int n = 0; n < nl; ++n) {
       Lev& l = L[n];
-      const bool in_arena = n >= arena_l;
-      auto get = [&](int slot, long count) { return in_arena ? (T*)(arena + offs[n][slot]) : mem.alloc<T>(count); };
-      for (int a = 0; a < dm; ++a) l.b[a] = get(a, fsize(l.g, a));
-      l.phi = get(3, csize(l.g));
-      l.rhs = get(4, csize(l.g));
-      l.tmp = get(5, csize(l.g));
-      phi_off_l[n] = in_arena ? offs[n][3] : 0;
+      const bool in_work = n >= work_l;
+      for (int a = 0; a < dm; ++a) {
+        l.b[a] = in_work ? cnext : mem.alloc<T>(fsize(l.g, a));
+        if (in_work) cnext += (fsize(l.g, a) + 63) / 64 * 64;
+      }
+      l.phi = in_work ? work + work_off[n] : mem.alloc<T>(csize(l.g));
+      l.rhs = in_work ? l.phi + mac_span(l.g) : mem.alloc<T>(csize(l.g));
+      l.tmp = in_work ? l.phi + 2 * mac_span(l.g) : mem.alloc<T>(csize(l.g));
     }
   }
-  unsigned char* arena = nullptr;  // levels arena_l .. nl-1, as in StagMG
-  int arena_l = 0;
-  std::vector<long> lev_end, phi_off_l;
+  T* work = nullptr;
+  int work_l = 0;
+  std::vector<long> work_off;
+  int coarse_start(int cn) const {
+    int l0 = nl;
+    while (l0 > std::max(work_l, nl - COARSE_MAXL) &&
+           coarse_fits(L[l0 - 1].g, cn, mac_slots(L[l0 - 1].g), mac_slots_max<T>(dm),
+                       (work_off[l0 - 1] + 3 * mac_span(L[l0 - 1].g)) * (long)sizeof(T)))
+      --l0;
+    return l0;
+  }
   void set_coeffs(hipStream_t s, double* const* alpha64) {
     Lev& l0 = L[0];
     for (int a = 0; a < dm; ++a) {
@@ -1879,40 +1465,46 @@ struct MacMG {
   }
   MacCoarseArgs<T>* coarse_args = nullptr;
   int coarse_l0 = -1;
-  int coarse_nt = 512;
-  void build_coarse(int l0, int nt, hipStream_t s, DevMem& mem) {
+  int coarse_nt = COARSE_THREADS;
+  CoarseForm coarse_form = CoarseForm::lds;
+  void build_coarse(int cn, int nt, hipStream_t s, DevMem& mem) {
+    const int l0 = coarse_start(cn);
     coarse_l0 = l0;
     coarse_nt = nt;
     if (l0 >= nl) return;
-    MacCoarseArgs<T> A;
-    memset(&A, 0, sizeof(A));
-    A.l0 = l0;
-    A.nl = nl;
+    std::unique_ptr<MacCoarseArgs<T>> Ap(new MacCoarseArgs<T>);
+    MacCoarseArgs<T>& A = *Ap;
+    memset((void*)&A, 0, sizeof(A));
+    A.l0 = 0;
+    A.nl = nl - l0;
     A.nu_down = nu_down;
     A.nu_up = nu_up;
     A.nu_bottom = nu_bottom;
+    A.work = work;
+    coarse_form = coarse_kernel_form((work_off[l0] + 3 * mac_span(L[l0].g)) * (long)sizeof(T), mac_slots(L[l0].g), nt);
     for (int n = l0; n < nl; ++n) {
-      MacLevArgs<T>& a = A.L[n];
-      a.g = L[n].g;
+      MacLevArgs<T>& a = A.L[n - l0];
+      const Geo& gl = L[n].g;
+      a.g = gl;
       a.h2i = L[n].h2i;
-      for (int d = 0; d < 3; ++d) a.b[d] = L[n].b[d];
-      a.phi = L[n].phi;
-      a.rhs = L[n].rhs;
-      a.tmp = L[n].tmp;
-      a.dcell = make_dec(L[n].g.n[0], L[n].g.n[1]);
-      a.dcolor = make_dec_color(L[n].g.n[0], L[n].g.n[1]);
+      a.inplace = even_level(gl);
+      a.half = mac_slots(gl) / 2;
+      a.nc = (gl.n[0] + 1) / 2 * gl.n[1] * gl.n[2];
+      a.phi = (int)work_off[n];
+      a.span = (int)mac_span(gl);
+      for (int d = 0; d < dm; ++d) {
+        a.fnx[d] = fext(gl, d, 0);
+        a.fnxy[d] = a.fnx[d] * fext(gl, d, 1);
+        a.b[d] = L[n].b[d];
+      }
+      a.dcell = make_dec(gl.n[0], gl.n[1]);
+      a.dcolor = make_dec_color(gl.n[0], gl.n[1]);
     }
-    A.st = stage_info(arena, arena_l, lev_end, phi_off_l[l0], csize(L[l0].g) * (long)sizeof(T), l0);
     if (!coarse_args) coarse_args = mem.alloc<MacCoarseArgs<T>>(1);
     h2d(coarse_args, &A, sizeof(A), s);
   }
-  template <int DM>
-  void coarse(hipStream_t s, int l0) {
-    (void)l0;
-    const int nt = coarse_nt;
-    if (nt == 256) launch_blocks(s, 1, MacCoarseBlk<T, DM, 256>{coarse_args});
-    else if (nt == 512) launch_blocks(s, 1, MacCoarseBlk<T, DM, 512>{coarse_args});
-    else launch_blocks(s, 1, MacCoarseBlk<T, DM, 1024>{coarse_args});
+  void coarse(hipStream_t s) {
+    launch_mac_coarse<T>(s, dm, coarse_nt, coarse_form, coarse_args);
     check_launch();
   }
   template <int DM>
@@ -1926,7 +1518,7 @@ struct MacMG {
           Lev& c = L[n + 1];
           launch(s, csize(c.g), MacResidRestrictFn<T, DM>{f.g, c.g, {f.b[0], f.b[1], f.b[2]}, f.h2i, f.phi, f.rhs, c.rhs, make_dec(c.g.n[0], c.g.n[1]), c.phi});
         }
-        coarse<DM>(s, l0);
+        coarse(s);
         for (int n = l0 - 1; n >= 0; --n) {
           launch(s, csize(L[n].g), MacProlongFn<T>{L[n].g, L[n + 1].g, L[n].phi, L[n + 1].phi, make_dec(L[n].g.n[0], L[n].g.n[1])});
           gs<DM>(s, n, nu_up);
@@ -2045,7 +1637,7 @@ __global__ void k_lsq_solve(LsqDev G, int i, double* __restrict__ coef) {
 struct Tune {
   int coarse_n = 8;         // staggered levels with every n_d <= coarse_n run in one workgroup
   int mac_coarse_n = 8;     // the same for the MAC hierarchy
-  int coarse_threads = 512; // threads of that workgroup
+  int coarse_threads = 1024; // threads of that workgroup
   int red_blocks = 1024;    // workgroups of an inner-product launch
   int graphs = 0;           // HIP-graph replay of Arnoldi steps and preconditioner applications
   int rows_n = 0;           // staggered levels with n_x >= rows_n smooth and apply by rows (0: never)
@@ -3120,10 +2712,10 @@ static void apply_tune(Ctx& c, const Tune& t) {
   c.use_graphs = t.graphs == 1 && !c.batch;  // batched solves leave the host between steps
   c.graph_failed = false;
   auto stag = [&](auto& mg) {
-    mg.build_coarse(coarse_level(mg.L[0].g, mg.nl, t.coarse_n), t.coarse_threads, c.s, c.mem);
+    mg.build_coarse(t.coarse_n, t.coarse_threads, c.s, c.mem);
     mg.rows_n = t.rows_n;
   };
-  auto mac = [&](auto& mm) { mm.build_coarse(coarse_level(mm.L[0].g, mm.nl, t.mac_coarse_n), t.coarse_threads, c.s, c.mem); };
+  auto mac = [&](auto& mm) { mm.build_coarse(t.mac_coarse_n, t.coarse_threads, c.s, c.mem); };
   if (c.d.precision == LMFHD_MIXED) {
     stag(c.mg32);
     mac(c.mac32);

@@ -355,31 +355,6 @@ HD bool decode_color(long t, const Dec& D, int par, int& i, int& j, int& k) {
   i = 2 * ih + ((par + j + k) & 1);
   return i < D.nx;
 }
-// L phi (mode 0) or rhs - L phi (mode 1) on every face of component a; zero on wall faces
-template <typename T, int VT, int DM>
-struct ApplyFn {
-  Geo g;
-  Coefs<T> C;
-  T* phi[3];
-  const T* rhs;
-  T* out;
-  int a;
-  Dec dc;
-  int mode;
-  // the component through by_comp: with a runtime component the coarse-level kernels indexed
-  // the functor's arrays dynamically and kept it in scratch memory
-  HD void operator()(long t) const {
-    int i, j, k;
-    decode3(t, dc, i, j, k);
-    by_comp<DM>(a, [&](const int ac) __attribute__((always_inline)) {
-      const int I[3] = {i, j, k};
-      if (wall_face(g, ac, I[ac])) { out[t] = T(0); return; }
-      const T L = lphi<T, VT, DM>(g, C, phi, ac, i, j, k, nullptr);
-      out[t] = mode == 0 ? L : rhs[t] - L;
-    });
-  }
-};
-
 // face (i,j,k) exists for component a
 HD bool face_in(const Geo& g, int a, int i, int j, int k) {
   return i < fext(g, a, 0) && j < fext(g, a, 1) && k < fext(g, a, 2);
@@ -809,65 +784,11 @@ struct RestrictFn {
   }
 };
 
-// prolongation-add of component a (stag_mg_solver.f90:1365-1628), one fine face per item, natural
-// storage (the one-workgroup coarse levels)
-template <typename T, int DM>
-struct ProlongFn {
-  using value_type = T;
-  Geo gf, gc;
-  T* f;
-  const T* c;
-  int a;
-  Dec dc;
-  HD void operator()(long t) const {
-    int i, j, k;
-    decode3(t, dc, i, j, k);
-    by_comp<DM>(a, [&](const int ac) __attribute__((always_inline)) { st(f, (unsigned)t, eval(i, j, k, t, ac)); });
-  }
-  // the new value of face (i,j,k), stored at offset t of f (wall faces unchanged); every
-  // operand is loaded before any is used, and the even and odd sums are both formed, so the
-  // loads are in flight together
-  HD T eval(int i, int j, int k, long t, const int a) const {
-    const int I[3] = {i, j, k};
-    const T old = ld(f, (unsigned)t);
-    int tb[2];
-    transverse(a, tb[0], tb[1]);
-    int C0[3] = {i / 2, j / 2, k / 2};
-    int off[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) off[d] = (I[d] % 2 == 0) ? -1 : 1;
-    auto P = [&](int na, int nb, int nc) {
-      int J[3] = {C0[0], C0[1], C0[2]};
-      J[a] += na;
-      J[tb[0]] += nb;
-      if (DM == 3) J[tb[1]] += nc;
-      return vel_at(c, gc, a, J[0], J[1], J[2]);
-    };
-    const int ob = off[tb[0]], oc = DM == 3 ? off[tb[1]] : 0;
-    const bool even = I[a] % 2 == 0;
-    T add;
-    if (DM == 3) {
-      const T p000 = P(0, 0, 0), p0b0 = P(0, ob, 0), p00c = P(0, 0, oc), p0bc = P(0, ob, oc);
-      const T p100 = P(1, 0, 0), p1b0 = P(1, ob, 0), p10c = P(1, 0, oc), p1bc = P(1, ob, oc);
-      const T se = T(9.0 / 16.0) * p000 + T(3.0 / 16.0) * p0b0 + T(3.0 / 16.0) * p00c + T(1.0 / 16.0) * p0bc;
-      const T so = T(9.0 / 32.0) * p000 + T(3.0 / 32.0) * p0b0 + T(3.0 / 32.0) * p00c + T(1.0 / 32.0) * p0bc +
-                   T(9.0 / 32.0) * p100 + T(3.0 / 32.0) * p1b0 + T(3.0 / 32.0) * p10c + T(1.0 / 32.0) * p1bc;
-      add = even ? se : so;
-    } else {
-      const T p000 = P(0, 0, 0), p0b0 = P(0, ob, 0), p100 = P(1, 0, 0), p1b0 = P(1, ob, 0);
-      const T se = T(0.75) * p000 + T(0.25) * p0b0;
-      const T so = T(0.375) * p000 + T(0.125) * p0b0 + T(0.375) * p100 + T(0.125) * p1b0;
-      add = even ? se : so;
-    }
-    return wall_face(gf, a, I[a]) ? old : old + add;
-  }
-};
-
-// Prolongation-add from the coarse side: one thread per coarse face (I,J,K) of component a adds
-// to the 2^dm fine faces (2I, 2J+dj, 2K+dk) and, below the last coarse face along a, to the
+// Prolongation-add (stag_mg_solver.f90:1365-1628) from the coarse side: one thread per coarse
+// face (I,J,K) of component a adds to the 2^dm fine faces (2I, 2J+dj, 2K+dk) and, below the last coarse face along a, to the
 // 2^dm faces (2I+1, ...) between I and I+1.  Those fine faces use the coarse values at I, I+1
-// along a and J-1..J+1, K-1..K+1 across it, loaded once here (18 in 3-D) where ProlongFn loads
-// 8 per fine face; each fine face gets ProlongFn's sums in ProlongFn's order.
+// along a and J-1..J+1, K-1..K+1 across it, loaded once here (18 in 3-D); a thread per fine face
+// would load 8 each.
 template <typename T, int DM>
 struct ProlongCFn {
   Geo gf, gc;
