@@ -293,116 +293,177 @@ __global__ void __launch_bounds__(256) k_maxpy(double* __restrict__ y, const dou
   y[e] = y[e] + sgn * s;
 }
 
-// The fused Gram-Schmidt passes of the Arnoldi step (grid-stride over the nb partial blocks of
-// k_mdot, partial sums part[PART(b, q)] reduced by k_red_final in a fixed order):
-//   k_mdot_self:  part_q = <w, V_q> for q < nv and part_nv = <w, w> (nv + 1 <= RED_NV);
-//   k_maxpy_dot:  w -= sum_q coef[q] V_q, then part_q = <w_new, V_q> for q < nv;
-//   k_maxpy_norm: unless *skip, w -= sum_q coef[q] V_q; part_0 = <w, w> of the result.
-// Inner products carry the Stokes-vector weights of element e0 + e.
-template <int NV>
-__global__ void __launch_bounds__(256) k_mdot_self(const double* __restrict__ w, const double* __restrict__ V,
-                                                   long vstride, int nv, VecLayout L, long n, long e0,
-                                                   double* __restrict__ part) {
-  double acc[NV + 1];
-#pragma unroll
-  for (int q = 0; q <= NV; ++q) acc[q] = 0.0;
-  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
-    const double x = w[e];
-    const double we = x * L.weight(e0 + e);
-#pragma unroll
-    for (int q = 0; q < NV; ++q) acc[q] += we * V[(q < nv ? q : nv - 1) * vstride + e];
-    acc[NV] += we * x;
-  }
-  __shared__ double sh[NV + 1][4];
+// The Arnoldi step's two Gram-Schmidt passes over nv = NV <= RED_NV - 1 basis vectors, three sweeps
+// and two one-workgroup reductions:
+//   k_gs_dot:     part_q = <w, V_q> for q < nv, part_nv = <w, w>;
+//   k_gs_dgks:    h1, |w|^2 and the second pass's flag *skip;
+//   k_gs_update:  w -= sum_q h1[q] V_q, then the same products of the result;
+//   k_gs_lsq:     h2 (0 with *skip), |w''| = sqrt(|w'|^2 - |h2|^2), the Givens column;
+//   k_gs_scale:   V_i = (w - sum_q h2[q] V_q) / |w''|.
+// Inner products carry the Stokes-vector weights.  They are bound by memory: nv + 1 vectors read
+// per sweep.  Two elements per lane (16-byte loads; the basis vectors start on multiples of 32
+// elements) and the exact number of vectors as a template argument: with 16 slots and a test per
+// slot the update ran at 3.1 TB/s at 256^3 (11.5 vectors on average), now at 4.9 (the products 5.8).  The norm by Pythagoras needs
+// no sweep of its own, since h2 is what the first pass left: of the order of the rounding of w,
+// so |h2|^2 is far below |w'|^2; where it is not (a step that has lost all of w), the step is
+// repeated with the norm formed (gs_repair).  The update walks the vectors from the end, so that
+// it starts on what the products' sweep left in the Infinity Cache.
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+template <int N>
+__device__ __forceinline__ void gs_partials(const double* acc, double* __restrict__ part) {
+  __shared__ double sh[N][4];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
-  for (int q = 0; q <= NV; ++q) {
+  for (int q = 0; q < N; ++q) {
     const double v = wave_sum(acc[q]);
     if (lane == 0) sh[q][wid] = v;
   }
   __syncthreads();
-  if ((int)threadIdx.x <= nv) {
-    const int q = threadIdx.x == nv ? NV : threadIdx.x;
-    part[PART(blockIdx.x, threadIdx.x)] = ((sh[q][0] + sh[q][1]) + sh[q][2]) + sh[q][3];
-  }
-}
-template <int NV>
-__global__ void __launch_bounds__(256) k_maxpy_dot(double* __restrict__ w, const double* __restrict__ V, long vstride,
-                                                   int nv, const double* __restrict__ coef, VecLayout L, long n,
-                                                   long e0, double* __restrict__ part) {
-  double c[NV], acc[NV];
-#pragma unroll
-  for (int q = 0; q < NV; ++q) {
-    c[q] = q < nv ? coef[q] : 0.0;
-    acc[q] = 0.0;
-  }
-  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
-    double v[NV];
-    double sum = 0.0;
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-      v[q] = V[(q < nv ? q : nv - 1) * vstride + e];
-      if (q < nv) sum += c[q] * v[q];
-    }
-    const double x = w[e] + (-1.0) * sum;
-    w[e] = x;
-    const double we = x * L.weight(e0 + e);
-#pragma unroll
-    for (int q = 0; q < NV; ++q) acc[q] += we * v[q];
-  }
-  __shared__ double sh[NV][4];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int q = 0; q < NV; ++q) {
-    const double r = wave_sum(acc[q]);
-    if (lane == 0) sh[q][wid] = r;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < nv) {
+  if ((int)threadIdx.x < N) {
     const int q = threadIdx.x;
     part[PART(blockIdx.x, q)] = ((sh[q][0] + sh[q][1]) + sh[q][2]) + sh[q][3];
   }
 }
 template <int NV>
-__global__ void __launch_bounds__(256) k_maxpy_norm(double* __restrict__ w, const double* __restrict__ V, long vstride,
-                                                    int nv, const double* __restrict__ coef, VecLayout L, long n,
-                                                    long e0, double* __restrict__ part,
-                                                    const double* __restrict__ skip) {
-  const bool upd = !(skip && skip[0] != 0.0);
-  double c[NV];
+__global__ void __launch_bounds__(256) k_gs_dot(const double* __restrict__ w, const double* __restrict__ V, long vs,
+                                                VecLayout L, long n, double* __restrict__ part) {
+  double acc[NV + 1];
 #pragma unroll
-  for (int q = 0; q < NV; ++q) c[q] = q < nv ? coef[q] : 0.0;
-  double acc = 0.0;
-  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
-    double x = w[e];
-    if (upd) {
-      // every load unconditional (q >= nv re-reads vector nv-1 from cache), so the loads of an
-      // element are in flight together; the sum takes the q < nv terms as before
-      double v[NV];
+  for (int q = 0; q <= NV; ++q) acc[q] = 0.0;
+  const long np = n >> 1;
+  for (long p = (long)blockIdx.x * 256 + threadIdx.x; p < np; p += (long)gridDim.x * 256) {
+    const dbl2 x = *(const dbl2*)(w + 2 * p);
+    dbl2 v[NV];
 #pragma unroll
-      for (int q = 0; q < NV; ++q) v[q] = V[(q < nv ? q : nv - 1) * vstride + e];
-      double sum = 0.0;
+    for (int q = 0; q < NV; ++q) v[q] = *(const dbl2*)(V + q * vs + 2 * p);
+    const double a = x.x * L.weight(2 * p), b = x.y * L.weight(2 * p + 1);
 #pragma unroll
-      for (int q = 0; q < NV; ++q)
-        if (q < nv) sum += c[q] * v[q];
-      x = x + (-1.0) * sum;
-      w[e] = x;
+    for (int q = 0; q < NV; ++q) {
+      acc[q] += a * v[q].x;
+      acc[q] += b * v[q].y;
     }
-    acc += (x * L.weight(e0 + e)) * x;
+    acc[NV] += a * x.x;
+    acc[NV] += b * x.y;
   }
-  __shared__ double sh[4];
-  const double r = wave_sum(acc);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = r;
-  __syncthreads();
-  if (threadIdx.x == 0) part[PART(blockIdx.x, 0)] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+    const double x = w[n - 1], a = x * L.weight(n - 1);
+#pragma unroll
+    for (int q = 0; q < NV; ++q) acc[q] += a * V[q * vs + n - 1];
+    acc[NV] += a * x;
+  }
+  gs_partials<NV + 1>(acc, part);
 }
-
+template <int NV>
+__global__ void __launch_bounds__(256) k_gs_update(double* __restrict__ w, const double* __restrict__ V, long vs,
+                                                   const double* __restrict__ h, VecLayout L, long n,
+                                                   double* __restrict__ part) {
+  double c[NV], acc[NV + 1];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) c[q] = h[q];
+#pragma unroll
+  for (int q = 0; q <= NV; ++q) acc[q] = 0.0;
+  const long np = n >> 1;
+  for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < np; t += (long)gridDim.x * 256) {
+    const long p = np - 1 - t;
+    dbl2 x = *(const dbl2*)(w + 2 * p);
+    dbl2 v[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) v[q] = *(const dbl2*)(V + q * vs + 2 * p);
+    double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      s0 += c[q] * v[q].x;
+      s1 += c[q] * v[q].y;
+    }
+    x.x -= s0;
+    x.y -= s1;
+    *(dbl2*)(w + 2 * p) = x;
+    const double a = x.x * L.weight(2 * p), b = x.y * L.weight(2 * p + 1);
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      acc[q] += a * v[q].x;
+      acc[q] += b * v[q].y;
+    }
+    acc[NV] += a * x.x;
+    acc[NV] += b * x.y;
+  }
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+    double sum = 0.0;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) sum += c[q] * V[q * vs + n - 1];
+    const double x = w[n - 1] - sum, a = x * L.weight(n - 1);
+    w[n - 1] = x;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) acc[q] += a * V[q * vs + n - 1];
+    acc[NV] += a * x;
+  }
+  gs_partials<NV + 1>(acc, part);
+}
+template <int NV>
+__global__ void __launch_bounds__(256) k_gs_scale(double* __restrict__ out, const double* __restrict__ w,
+                                                  const double* __restrict__ V, long vs, const double* __restrict__ h,
+                                                  const double* __restrict__ nrm, const double* __restrict__ skip,
+                                                  long n) {
+  const long np = n >> 1;
+  const long p = (long)blockIdx.x * 256 + threadIdx.x;
+  if (p > np) return;
+  const double den = nrm[0];
+  const bool upd = skip[0] == 0.0;
+  if (p == np) {
+    if (!(n & 1)) return;
+    double sum = 0.0;
+    if (upd)
+      for (int q = 0; q < NV; ++q) sum += h[q] * V[q * vs + n - 1];
+    out[n - 1] = (w[n - 1] - sum) / den;
+    return;
+  }
+  dbl2 x = *(const dbl2*)(w + 2 * p);
+  if (upd) {
+    dbl2 v[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) v[q] = *(const dbl2*)(V + q * vs + 2 * p);
+    double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      s0 += h[q] * v[q].x;
+      s1 += h[q] * v[q].y;
+    }
+    x.x -= s0;
+    x.y -= s1;
+  }
+  x.x /= den;
+  x.y /= den;
+  *(dbl2*)(out + 2 * p) = x;
+}
+// out[q] = sum_b part[PART(b, q)], q < nv <= 16, by a workgroup of 1024: a wave per product
+__device__ __forceinline__ void gs_reduce(const double* __restrict__ part, int nb, int nv, double* __restrict__ out) {
+  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (q < nv) {
+    double s = 0.0;
+    for (int b = lane; b < nb; b += 64) s += part[PART(b, q)];
+    s = wave_sum(s);
+    if (lane == 0) out[q] = s;
+  }
+  __syncthreads();
+}
 // skip = 1 when |w - V h|^2 = wn2 - |h|^2 >= wn2 / 2 (no second Gram-Schmidt pass), else 0
 __global__ void k_dgks(const double* __restrict__ h, int nh, const double* __restrict__ wn2, double* __restrict__ skip) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   double hh = 0.0;
   for (int q = 0; q < nh; ++q) hh += h[q] * h[q];
   skip[0] = (wn2[0] - hh >= 0.5 * wn2[0]) ? 1.0 : 0.0;
+}
+
+__global__ void __launch_bounds__(1024) k_gs_dgks(const double* __restrict__ part, int nb, int nv,
+                                                  double* __restrict__ h1, double* __restrict__ skip) {
+  __shared__ double r[RED_NV];
+  gs_reduce(part, nb, nv + 1, r);
+  if ((int)threadIdx.x <= nv) h1[threadIdx.x] = r[threadIdx.x];
+  if (threadIdx.x == 0) {
+    double hh = 0.0;
+    for (int q = 0; q < nv; ++q) hh += r[q] * r[q];
+    skip[0] = (r[nv] - hh >= 0.5 * r[nv]) ? 1.0 : 0.0;
+  }
 }
 
 // dst = src / *den
@@ -495,71 +556,77 @@ struct Reducer {
     check_launch();
 #endif
   }
-  // Fused Gram-Schmidt passes of the Arnoldi step, weighted inner products, nv + 1 <= RED_NV:
-  // out[q] = <w, V_q> (q < nv), out[nv] = <w, w>
-  void mdot_self(const double* w, const double* V, long vstride, int nv, long n, double* out) {
+  // The sweeps of the Arnoldi step over nv < RED_NV basis vectors at a stride of vs elements (the
+  // kernels above; the one-workgroup reductions are the Arnoldi step's).  Vectors on 16-byte
+  // boundaries, vs even.
+#ifndef LMFHD_HOST_DEBUG
+  template <class F>
+  static void by_nv(int nv, F&& f) {
+    switch (nv) {
+#define LMFHD_NV(N) case N: f(std::integral_constant<int, N>{}); break;
+      LMFHD_NV(1) LMFHD_NV(2) LMFHD_NV(3) LMFHD_NV(4) LMFHD_NV(5) LMFHD_NV(6) LMFHD_NV(7) LMFHD_NV(8)
+      LMFHD_NV(9) LMFHD_NV(10) LMFHD_NV(11) LMFHD_NV(12) LMFHD_NV(13) LMFHD_NV(14) LMFHD_NV(15)
+#undef LMFHD_NV
+      default: set_err("internal: Gram-Schmidt over %d vectors", nv); throw Fail{LMFHD_E_ARG};
+    }
+  }
+  // workgroups of a sweep over n elements, two per lane
+  int gs_blocks(long n) const { return (int)std::min<long>(max_blocks, std::max<long>(1, (n / 2 + 255) / 256)); }
+#endif
+  // products of w with V_0 .. V_nv-1 and itself; h1[q], h1[nv] = |w|^2, the second pass's flag
+  void gs_dot(const double* w, const double* V, long vs, int nv, long n, double* h1, double* skip) {
 #ifdef LMFHD_HOST_DEBUG
+    double hh = 0.0;
     for (int q = 0; q <= nv; ++q) {
       double acc = 0.0;
-      for (long e = 0; e < n; ++e) acc += (w[e] * L.weight(e)) * (q < nv ? V[q * vstride + e] : w[e]);
-      out[q] = acc;
+      for (long e = 0; e < n; ++e) acc += (w[e] * L.weight(e)) * (q < nv ? V[q * vs + e] : w[e]);
+      h1[q] = acc;
+      if (q < nv) hh += acc * acc;
     }
+    skip[0] = (h1[nv] - hh >= 0.5 * h1[nv]) ? 1.0 : 0.0;
 #else
-    const int nb = nblocks(n);
-    if (nv <= 1) hipLaunchKernelGGL(k_mdot_self<1>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, L, n, 0L, part);
-    else if (nv <= 4) hipLaunchKernelGGL(k_mdot_self<4>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, L, n, 0L, part);
-    else if (nv <= 8) hipLaunchKernelGGL(k_mdot_self<8>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, L, n, 0L, part);
-    else hipLaunchKernelGGL(k_mdot_self<16>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, L, n, 0L, part);
-    hipLaunchKernelGGL(k_red_final, dim3(1), dim3(256), 0, s, part, nb, nv + 1, 0, out, nullptr);
+    const int nb = gs_blocks(n);
+    by_nv(nv, [&](auto N) { hipLaunchKernelGGL(k_gs_dot<decltype(N)::value>, dim3(nb), dim3(256), 0, s, w, V, vs, L, n, part); });
+    hipLaunchKernelGGL(k_gs_dgks, dim3(1), dim3(1024), 0, s, (const double*)part, nb, nv, h1, skip);
     check_launch();
 #endif
   }
-  // w -= sum_q coef[q] V_q; out[q] = <w_new, V_q>, or 0 when *skip_out != 0
-  void maxpy_dot(double* w, const double* V, long vstride, int nv, const double* coef, long n, double* out,
-                 const double* skip_out) {
+  // w -= sum_q h[q] V_q, then the same products of the result: on the device left as partial sums
+  // for the Givens column's kernel (returns their number), in the host build in prod[0 .. nv]
+  int gs_update(double* w, const double* V, long vs, int nv, const double* h, long n, double* prod) {
 #ifdef LMFHD_HOST_DEBUG
     for (long e = 0; e < n; ++e) {
       double sum = 0.0;
-      for (int q = 0; q < nv; ++q) sum += coef[q] * V[q * vstride + e];
-      w[e] = w[e] + (-1.0) * sum;
+      for (int q = 0; q < nv; ++q) sum += h[q] * V[q * vs + e];
+      w[e] = w[e] - sum;
     }
-    for (int q = 0; q < nv; ++q) {
+    for (int q = 0; q <= nv; ++q) {
       double acc = 0.0;
-      for (long e = 0; e < n; ++e) acc += (w[e] * L.weight(e)) * V[q * vstride + e];
-      out[q] = (skip_out && skip_out[0] != 0.0) ? 0.0 : acc;
+      for (long e = 0; e < n; ++e) acc += (w[e] * L.weight(e)) * (q < nv ? V[q * vs + e] : w[e]);
+      prod[q] = acc;
     }
+    return 0;
 #else
-    const int nb = nblocks(n);
-    if (nv <= 1) hipLaunchKernelGGL(k_maxpy_dot<1>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part);
-    else if (nv <= 4) hipLaunchKernelGGL(k_maxpy_dot<4>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part);
-    else if (nv <= 8) hipLaunchKernelGGL(k_maxpy_dot<8>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part);
-    else hipLaunchKernelGGL(k_maxpy_dot<16>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part);
-    hipLaunchKernelGGL(k_red_final, dim3(1), dim3(256), 0, s, part, nb, nv, 0, out, skip_out);
+    (void)prod;
+    const int nb = gs_blocks(n);
+    by_nv(nv, [&](auto N) { hipLaunchKernelGGL(k_gs_update<decltype(N)::value>, dim3(nb), dim3(256), 0, s, w, V, vs, h, L, n, part); });
     check_launch();
+    return nb;
 #endif
   }
-  // unless *skip: w -= sum_q coef[q] V_q; *nrm = sqrt <w, w>
-  void maxpy_norm(double* w, const double* V, long vstride, int nv, const double* coef, long n, double* nrm,
-                  const double* skip) {
+  // out = (w - sum_q h[q] V_q) / *nrm, the sum only where *skip is 0
+  void gs_scale(double* out, const double* w, const double* V, long vs, int nv, const double* h, const double* nrm,
+                const double* skip, long n) {
 #ifdef LMFHD_HOST_DEBUG
-    const bool upd = !(skip && skip[0] != 0.0);
-    double acc = 0.0;
     for (long e = 0; e < n; ++e) {
-      if (upd) {
-        double sum = 0.0;
-        for (int q = 0; q < nv; ++q) sum += coef[q] * V[q * vstride + e];
-        w[e] = w[e] + (-1.0) * sum;
-      }
-      acc += (w[e] * L.weight(e)) * w[e];
+      double sum = 0.0;
+      if (skip[0] == 0.0)
+        for (int q = 0; q < nv; ++q) sum += h[q] * V[q * vs + e];
+      out[e] = (w[e] - sum) / nrm[0];
     }
-    nrm[0] = std::sqrt(acc);
 #else
-    const int nb = nblocks(n);
-    if (nv <= 1) hipLaunchKernelGGL(k_maxpy_norm<1>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part, skip);
-    else if (nv <= 4) hipLaunchKernelGGL(k_maxpy_norm<4>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part, skip);
-    else if (nv <= 8) hipLaunchKernelGGL(k_maxpy_norm<8>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part, skip);
-    else hipLaunchKernelGGL(k_maxpy_norm<16>, dim3(nb), dim3(256), 0, s, w, V, vstride, nv, coef, L, n, 0L, part, skip);
-    hipLaunchKernelGGL(k_red_final, dim3(1), dim3(256), 0, s, part, nb, 1, 1, nrm, nullptr);
+    const long nb = (n / 2 + 1 + 255) / 256;
+    by_nv(nv, [&](auto N) { hipLaunchKernelGGL(k_gs_scale<decltype(N)::value>, dim3(nb), dim3(256), 0, s, out, w, V, vs, h, nrm, skip, n); });
     check_launch();
 #endif
   }
@@ -1563,7 +1630,8 @@ struct LsqDev {
   double* sn;
   double* sv;
   double* y;
-  double* stat;  // [0] |s(i+1)|, the residual estimate; [1] 1 when it passes the stop test; [2] H(i+1, i)
+  double* stat;  // [0] |s(i+1)|, the residual estimate; [1] 1 when it passes the stop test; [2] H(i+1, i);
+                 // [3] 1 when the step lost all of w and is to be repaired (gs_repair)
   double* thr;   // stop thresholds: [0] relative (rel_tol times the reference norm), [1] absolute
   int m;
   HD double& h(int r, int col) const { return H[(long)r * (m + 1) + col]; }
@@ -1581,6 +1649,20 @@ HD void rotmat_hd(double a, double b, double& cs, double& sn) {
     cs = 1.0 / sqrt(1.0 + t * t);
     sn = t * cs;
   }
+}
+// The column i from the second pass's products prod[0 .. i-1] and |w'|^2 = prod[i]: h2, |w''| by
+// Pythagoras, and whether it may be used (else stat[3] = 1 and the step waits for gs_repair)
+HD bool lsq_norm_hd(const LsqDev& G, int i, const double* prod, const double* skip, double* h2, double* nrm) {
+  double hh = 0.0;
+  for (int q = 0; q < i; ++q) {
+    h2[q] = skip[0] != 0.0 ? 0.0 : prod[q];
+    hh += h2[q] * h2[q];
+  }
+  const double n2 = prod[i] - hh;
+  nrm[0] = sqrt(n2);
+  const bool lost = n2 < 0.25 * prod[i];
+  G.stat[3] = lost ? 1.0 : 0.0;
+  return !lost;
 }
 // least_squares (gmres.f90:531-566) for column i: H(1..i, i) = h1 + h2 (the two Gram-Schmidt
 // passes), H(i+1, i) = |w|; earlier rotations, the new rotation, s, the estimate and the test
@@ -1623,6 +1705,53 @@ HD void lsq_solve_hd(const LsqDev& G, int i, double* coef) {
 __global__ void k_lsq_column(LsqDev G, int i, const double* __restrict__ h1, const double* __restrict__ h2,
                              const double* __restrict__ nrm) {
   if (threadIdx.x == 0 && blockIdx.x == 0) lsq_column_hd(G, i, h1, h2, nrm);
+}
+// the reduction of k_gs_update's partial sums, then lsq_norm_hd and the Givens column.  The column
+// and the rotations are brought to LDS in one step, so that the one thread's chain of i rotations
+// waits for LDS instead of memory
+__global__ void __launch_bounds__(1024) k_gs_lsq(LsqDev G, int i, const double* __restrict__ part, int nb,
+                                                 const double* __restrict__ h1, double* __restrict__ h2,
+                                                 double* __restrict__ nrm, const double* __restrict__ skip) {
+  __shared__ double r[RED_NV], a1[RED_NV], a2[RED_NV], cs[RED_NV + 2], sn[RED_NV + 2], sv[2], col[RED_NV + 2], nr[1];
+  const int t = threadIdx.x;
+  if (t < i) a1[t] = h1[t];
+  if (t >= 64 && t < 64 + i) {
+    cs[t - 63] = G.cs[t - 63];
+    sn[t - 63] = G.sn[t - 63];
+  }
+  if (t == 128) sv[0] = G.sv[i];
+  gs_reduce(part, nb, i + 1, r);
+  if (t == 0) {
+    const double sk = skip[0];
+    if (lsq_norm_hd(G, i, r, &sk, a2, nr)) {
+      // lsq_column_hd on the copies: H with one column, s with its entry i
+      LsqDev C = G;
+      for (int q = 1; q <= i; ++q) col[q] = a1[q - 1] + a2[q - 1];
+      col[i + 1] = nr[0];
+      for (int k = 1; k <= i - 1; ++k) {
+        const double u = cs[k] * col[k] + sn[k] * col[k + 1];
+        col[k + 1] = -sn[k] * col[k] + cs[k] * col[k + 1];
+        col[k] = u;
+      }
+      rotmat_hd(col[i], col[i + 1], cs[i], sn[i]);
+      const double u = cs[i] * sv[0];
+      const double sv1 = -sn[i] * sv[0];
+      C.sv[i + 1] = sv1;
+      C.sv[i] = u;
+      C.cs[i] = cs[i];
+      C.sn[i] = sn[i];
+      col[i] = cs[i] * col[i] + sn[i] * col[i + 1];
+      col[i + 1] = 0.0;
+      const double est = fabs(sv1);
+      G.stat[0] = est;
+      G.stat[1] = (est <= G.thr[0] || est <= G.thr[1]) ? 1.0 : 0.0;
+      G.stat[2] = nr[0];
+    }
+    nrm[0] = nr[0];
+  }
+  __syncthreads();
+  if (t < i) h2[t] = a2[t];
+  if (t >= 1 && t <= i + 1) G.h(t, i) = col[t];
 }
 __global__ void k_lsq_init(LsqDev G, const double* __restrict__ nrm, double thr_rel, double thr_abs) {
   if (threadIdx.x == 0 && blockIdx.x == 0) lsq_init_hd(G, nrm, thr_rel, thr_abs);
@@ -1687,8 +1816,9 @@ struct Ctx {
   float* macrhs32 = nullptr;
   // Stokes vectors (FP64): Krylov basis and work
   int m = 5;
-  double* V = nullptr;  // (m+1) * vlen
-  double* Z = nullptr;  // m * vlen (FGMRES)
+  long vs = 0;          // stride of the basis vectors: vlen rounded up to 32 elements
+  double* V = nullptr;  // (m+1) * vs
+  double* Z = nullptr;  // m * vs (FGMRES)
   double* r = nullptr;
   double* w = nullptr;
   double* tmp = nullptr;
@@ -2373,36 +2503,54 @@ static void arnoldi(Ctx& c, double* w, int i) {
   // for the orthonormal basis).  The reference orthogonalises by modified Gram-Schmidt
   // (gmres.f90:352-372).
   double* nrm = c.s_nrm();
-  if (i + 1 <= RED_NV) {
-    // the same passes with the dot products folded into the sweeps that already read the
-    // vectors: <w, V>, |w|^2 together; the first update with the second pass's dot products;
-    // the second update (when needed) with the norm. Same sums in the same order.
-    c.R.mdot_self(w, c.V, c.vlen, i, c.vlen, h1);  // h1[i] = |w|^2
-    dgks(s, h1, i, h1 + i, skip);
-    c.R.maxpy_dot(w, c.V, c.vlen, i, h1, c.vlen, h2, skip);
-    c.R.maxpy_norm(w, c.V, c.vlen, i, h2, c.vlen, nrm, skip);
-  } else {
-    c.R.mdot(w, w, 0, 1, c.vlen, true, wn2);
-    for (int pass = 0; pass < 2; ++pass) {
-      double* h = pass == 0 ? h1 : h2;
-      const double* sk = pass == 0 ? nullptr : skip;
-      for (int q0 = 0; q0 < i; q0 += RED_NV) {
-        const int nv = std::min(RED_NV, i - q0);
-        c.R.mdot(w, c.V + (long)q0 * c.vlen, c.vlen, nv, c.vlen, true, h + q0, false, 0, sk);
-      }
-      maxpy(s, w, c.V, c.vlen, i, h, -1.0, c.vlen, sk);
-      if (pass == 0) dgks(s, h1, i, wn2, skip);
-    }
-    c.R.mdot(w, w, 0, 1, c.vlen, true, nrm, true);
+  if (i < RED_NV) {
+    c.R.gs_dot(w, c.V, c.vs, i, c.vlen, h1, skip);  // h1[i] = |w|^2
+#ifdef LMFHD_HOST_DEBUG
+    double prod[RED_NV];
+    c.R.gs_update(w, c.V, c.vs, i, h1, c.vlen, prod);
+    if (lsq_norm_hd(c.G, i, prod, skip, h2, nrm)) lsq_column_hd(c.G, i, h1, h2, nrm);
+#else
+    const int nb = c.R.gs_update(w, c.V, c.vs, i, h1, c.vlen, nullptr);
+    hipLaunchKernelGGL(k_gs_lsq, dim3(1), dim3(1024), 0, s, c.G, i, (const double*)c.R.part, nb, (const double*)h1, h2,
+                       nrm, (const double*)skip);
+    check_launch();
+#endif
+    c.R.gs_scale(c.V + (long)i * c.vs, w, c.V, c.vs, i, h2, nrm, skip, c.vlen);
+    return;
   }
-  scale_div(s, c.V + (long)i * c.vlen, w, nrm, c.vlen);
+  c.R.mdot(w, w, 0, 1, c.vlen, true, wn2);
+  for (int pass = 0; pass < 2; ++pass) {
+    double* h = pass == 0 ? h1 : h2;
+    const double* sk = pass == 0 ? nullptr : skip;
+    for (int q0 = 0; q0 < i; q0 += RED_NV) {
+      const int nv = std::min(RED_NV, i - q0);
+      c.R.mdot(w, c.V + (long)q0 * c.vs, c.vs, nv, c.vlen, true, h + q0, false, 0, sk);
+    }
+    maxpy(s, w, c.V, c.vs, i, h, -1.0, c.vlen, sk);
+    if (pass == 0) dgks(s, h1, i, wn2, skip);
+  }
+  c.R.mdot(w, w, 0, 1, c.vlen, true, nrm, true);
+  scale_div(s, c.V + (long)i * c.vs, w, nrm, c.vlen);
+  lsq_column(c, i);
+}
+// the end of an Arnoldi step whose w' the second pass reduced by more than half of |w'|^2: the
+// update applied, the norm formed, then the Givens column (the step's stat[3] asks for it)
+static void gs_repair(Ctx& c, double* w, int i) {
+  maxpy(c.s, w, c.V, c.vs, i, c.s_h2(), -1.0, c.vlen);
+  c.R.mdot(w, w, 0, 1, c.vlen, true, c.s_nrm(), true);
+  scale_div(c.s, c.V + (long)i * c.vs, w, c.s_nrm(), c.vlen);
   lsq_column(c, i);
 }
 
 static bool finite(double v) { return std::isfinite(v); }
 
-// status of the last Givens column on the host: {|s(i+1)|, stop flag, H(i+1, i)}
-static void lsq_status(Ctx& c, double* st) { d2h(st, c.G.stat, 3 * sizeof(double), c.s); }
+// status of Arnoldi step i (on w = c.w) on the host: {|s(i+1)|, stop flag, H(i+1, i), repair flag}
+static void lsq_status(Ctx& c, int i, double* st) {
+  d2h(st, c.G.stat, 4 * sizeof(double), c.s);
+  if (st[3] == 0.0) return;
+  gs_repair(c, c.w, i);
+  d2h(st, c.G.stat, 3 * sizeof(double), c.s);
+}
 
 // gmres (gmres.f90:32-621), left preconditioning, scale_factor = 1
 static int gmres_left(Ctx& c, const double* b, double* x, lmfhd_stats* st) {
@@ -2435,7 +2583,7 @@ static int gmres_left(Ctx& c, const double* b, double* x, lmfhd_stats* st) {
     S.converged = 1;
     return finish(LMFHD_OK);
   }
-  double stat[3];
+  double stat[4];
   while (true) {
     apply_matrix(c, x, c.tmp);
     S.n_matrix++;
@@ -2460,7 +2608,7 @@ static int gmres_left(Ctx& c, const double* b, double* x, lmfhd_stats* st) {
     for (int i = 1; i <= m; ++i) {
       total_iter++;
       i_copy = i;
-      double* Vi = c.V + (long)(i - 1) * c.vlen;
+      double* Vi = c.V + (long)(i - 1) * c.vs;
       run_graphed(c, 1, i, Vi, nullptr, [&]() {
         apply_matrix(c, Vi, c.tmp);
         precon_step(c, c.tmp, c.w);
@@ -2468,7 +2616,7 @@ static int gmres_left(Ctx& c, const double* b, double* x, lmfhd_stats* st) {
       });
       S.n_matrix++;
       S.n_precon++;
-      lsq_status(c, stat);
+      lsq_status(c, i, stat);
       if (!finite(stat[2])) { set_err("non-finite Arnoldi norm"); return finish(LMFHD_E_NAN); }
       if (stat[2] == 0.0) { set_err("gmres: error in orthogonalization"); return finish(LMFHD_E_BREAKDOWN); }
       if (nh < 256) S.resid_hist[nh++] = stat[0];
@@ -2476,7 +2624,7 @@ static int gmres_left(Ctx& c, const double* b, double* x, lmfhd_stats* st) {
       if (total_iter >= d.gmres_min_iter && stat[1] != 0.0) break;
     }
     lsq_solve(c, i_copy);
-    maxpy(s, x, c.V, c.vlen, i_copy, c.coef, 1.0, c.vlen);
+    maxpy(s, x, c.V, c.vs, i_copy, c.coef, 1.0, c.vlen);
   }
   return finish(LMFHD_OK);
 }
@@ -2518,7 +2666,7 @@ static int fgmres(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool want
     S.converged = 1;
     return finish(LMFHD_OK);
   }
-  double stat[3];
+  double stat[4];
   while (true) {
     apply_matrix(c, x, c.tmp);
     S.n_matrix++;
@@ -2538,8 +2686,8 @@ static int fgmres(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool want
     for (int i = 1; i <= m; ++i) {
       total_iter++;
       i_copy = i;
-      double* Vi = c.V + (long)(i - 1) * c.vlen;
-      double* Zi = c.Z + (long)(i - 1) * c.vlen;
+      double* Vi = c.V + (long)(i - 1) * c.vs;
+      double* Zi = c.Z + (long)(i - 1) * c.vs;
       run_graphed(c, 2, i, Vi, Zi, [&]() {
         precon_step(c, Vi, Zi);
         apply_matrix(c, Zi, c.w);
@@ -2547,7 +2695,7 @@ static int fgmres(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool want
       });
       S.n_precon++;
       S.n_matrix++;
-      lsq_status(c, stat);
+      lsq_status(c, i, stat);
       if (!finite(stat[2])) { set_err("non-finite Arnoldi norm"); return finish(LMFHD_E_NAN); }
       if (nh < 256) S.resid_hist[nh++] = stat[0];
       if (stat[2] == 0.0) break;  // exact solution in the Krylov space: finish this cycle
@@ -2555,7 +2703,7 @@ static int fgmres(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool want
       if (total_iter >= d.gmres_min_iter && stat[1] != 0.0) break;
     }
     lsq_solve(c, i_copy);
-    maxpy(s, x, c.Z, c.vlen, i_copy, c.coef, 1.0, c.vlen);
+    maxpy(s, x, c.Z, c.vs, i_copy, c.coef, 1.0, c.vlen);
   }
   return finish(LMFHD_OK);
 }
@@ -2770,6 +2918,7 @@ static void ctx_build(Ctx& c, const lmfhd_desc& d) {
   c.VL.off[1] = c.off[1];
   c.VL.off[2] = c.off[2];
   c.VL.off[3] = c.off[3];
+  c.vs = (c.vlen + 31) / 32 * 32;
   c.VL.off[4] = c.vlen;
   for (int dd = 0; dd < 3; ++dd) c.VL.n[dd] = c.g.n[dd];
   c.VL.dm = c.dm;
@@ -2794,8 +2943,8 @@ static void ctx_build(Ctx& c, const lmfhd_desc& d) {
     if (d.visc_schur_approx) c.macmu64.build(c.g, c.dx, d, c.mem);
   }
   if (d.visc_schur_approx) c.diaglap = c.mem.alloc<double>(c.vlen);
-  c.V = c.mem.alloc<double>((long)(c.m + 1) * c.vlen);
-  if (d.krylov == LMFHD_FGMRES) c.Z = c.mem.alloc<double>((long)c.m * c.vlen);
+  c.V = c.mem.alloc<double>((long)(c.m + 1) * c.vs);
+  if (d.krylov == LMFHD_FGMRES) c.Z = c.mem.alloc<double>((long)c.m * c.vs);
   c.r = c.mem.alloc<double>(c.vlen);
   c.w = c.mem.alloc<double>(c.vlen);
   c.tmp = c.mem.alloc<double>(c.vlen);
