@@ -1876,10 +1876,14 @@ struct Ctx {
 };
 
 // ------------------------------------------------------------------------------------------
-// apply_matrix: b = A x ; x wall faces zeroed in place first (apply_matrix.f90:71-115)
-static void apply_matrix(Ctx& c, double* x, double* b) {
+// apply_matrix (apply_matrix.f90:71-147): b = A x, wall faces of x counting as zero.  walls: what
+// they hold -- zero already (results of the preconditioner, combinations of them), to be zeroed in
+// place first as the reference does, or anything and left alone (a caller's const vector)
+enum class Walls { zero, clear, any };
+static void apply_matrix(Ctx& c, double* x, double* b, Walls walls) {
   hipStream_t s = c.s;
-  if (has_wall(c.g))
+  if (!has_wall(c.g)) walls = Walls::zero;
+  if (walls == Walls::clear)
     for (int a = 0; a < c.dm; ++a) {
       const int nx = fext(c.g, a, 0), ny = fext(c.g, a, 1);
       launch(s, c.nf[a], ZeroWallFacesFn<double>{c.g, c.u(x, a), a, make_dec(nx, ny)});
@@ -1921,13 +1925,23 @@ static void apply_matrix(Ctx& c, double* x, double* b) {
   }
   dispatch_vd(c.d.visc_type, c.dm, [&](auto V, auto D) {
     constexpr int VT = decltype(V)::value, DM = decltype(D)::value;
-    // one launch per component and one for the cells: measured faster than one column
-    // launch for everything (108 us against 137 us at 128^3)
-    for (int a = 0; a < c.dm; ++a) {
-      const int nx = fext(c.g, a, 0), ny = fext(c.g, a, 1);
-      launch(s, c.nf[a], AmFaceFn<VT, DM>{c.g, C, {c.u(x, 0), c.u(x, 1), c.dm == 3 ? c.u(x, 2) : c.u(x, 1)}, c.p(x), c.u(b, a), dxinv, a, make_dec(nx, ny)});
-    }
-    launch(s, c.nc, NegDivFn<DM>{c.g, {c.u(x, 0), c.u(x, 1), c.dm == 3 ? c.u(x, 2) : c.u(x, 1)}, c.p(b), dxinv, make_dec(c.g.n[0], c.g.n[1])});
+    auto go = [&](auto M) {
+      AmPosFn<VT, DM, decltype(M)::value> F;
+      F.g = c.g;
+      F.C = C;
+      F.dxinv = dxinv;
+      F.xp = c.p(x);
+      F.outp = c.p(b);
+      for (int a = 0; a < 3; ++a) {
+        F.xu[a] = c.u(x, a < DM ? a : DM - 1);
+        F.out[a] = c.u(b, a < DM ? a : DM - 1);
+      }
+      const ColShape cs = col_shape(c.g);
+      F.cx = cs.cx;
+      launch_cols(s, cs.ncols, cs.nz, cs.kc, F);
+    };
+    if (walls == Walls::any) go(std::integral_constant<int, 1>{});
+    else go(std::integral_constant<int, 0>{});
   });
   check_launch();
 }
@@ -2585,7 +2599,7 @@ static int gmres_left(Ctx& c, const double* b, double* x, lmfhd_stats* st) {
   }
   double stat[4];
   while (true) {
-    apply_matrix(c, x, c.tmp);
+    apply_matrix(c, x, c.tmp, Walls::clear);
     S.n_matrix++;
     rsub(s, c.tmp, b, c.vlen);  // tmp = b - A x
     norm_resid_stokes = vnorm(c, c.tmp);
@@ -2610,7 +2624,7 @@ static int gmres_left(Ctx& c, const double* b, double* x, lmfhd_stats* st) {
       i_copy = i;
       double* Vi = c.V + (long)(i - 1) * c.vs;
       run_graphed(c, 1, i, Vi, nullptr, [&]() {
-        apply_matrix(c, Vi, c.tmp);
+        apply_matrix(c, Vi, c.tmp, Walls::zero);
         precon_step(c, c.tmp, c.w);
         arnoldi(c, c.w, i);
       });
@@ -2668,7 +2682,7 @@ static int fgmres(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool want
   }
   double stat[4];
   while (true) {
-    apply_matrix(c, x, c.tmp);
+    apply_matrix(c, x, c.tmp, Walls::clear);
     S.n_matrix++;
     rsub(s, c.tmp, b, c.vlen);
     beta = vnorm(c, c.tmp);  // also left in s_tmp on the device
@@ -2690,7 +2704,7 @@ static int fgmres(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool want
       double* Zi = c.Z + (long)(i - 1) * c.vs;
       run_graphed(c, 2, i, Vi, Zi, [&]() {
         precon_step(c, Vi, Zi);
-        apply_matrix(c, Zi, c.w);
+        apply_matrix(c, Zi, c.w, Walls::zero);
         arnoldi(c, c.w, i);
       });
       S.n_precon++;
@@ -3597,7 +3611,7 @@ int lmfhd_apply_matrix_bc(lmfhd_ctx* x, const lmfhd_fab* x_u, const lmfhd_fab* x
   if (!upload_vec(c, x_u, x_p, c.io_a, h)) { set_err("x shape"); return LMFHD_E_ARG; }
   const double *dn, *dt;
   if (!upload_bc(c, vel_bc_n, vel_bc_t, dn, dt)) { set_err("vel_bc shape"); return LMFHD_E_ARG; }
-  apply_matrix(c, c.io_a, c.io_b);
+  apply_matrix(c, c.io_a, c.io_b, Walls::any);
   bc_lift(c, dn, dt, c.io_b, 1.0, -1.0);
   if (!download_vec(c, c.io_b, b_u, b_p, h)) { set_err("b shape"); return LMFHD_E_ARG; }
   return LMFHD_OK;
@@ -3680,7 +3694,7 @@ int lmfhd_apply_matrix(lmfhd_ctx* x, const lmfhd_fab* x_u, const lmfhd_fab* x_p,
   if (!c.have_coef) { set_err("coefficients not set"); return LMFHD_E_STATE; }
   std::vector<double> h;
   if (!upload_vec(c, x_u, x_p, c.io_a, h)) { set_err("x shape"); return LMFHD_E_ARG; }
-  apply_matrix(c, c.io_a, c.io_b);
+  apply_matrix(c, c.io_a, c.io_b, Walls::any);
   if (!download_vec(c, c.io_b, b_u, b_p, h)) { set_err("b shape"); return LMFHD_E_ARG; }
   return LMFHD_OK;
   API_END
@@ -3923,12 +3937,17 @@ int lmfhd_gmres_dev_batch(lmfhd_ctx** ctxs, int n, const double* const* b, doubl
   return first;
 }
 
+// a caller's vector as it is, or a copy of it where it overlaps the output b
+static double* apart(Ctx& c, const double* xv, const double* b) {
+  if (xv + c.vlen <= b || b + c.vlen <= xv) return const_cast<double*>(xv);
+  d2d(c.io_a, xv, c.vlen * sizeof(double), c.s);
+  return c.io_a;
+}
 int lmfhd_apply_matrix_dev(lmfhd_ctx* x, const double* xv, double* b) {
   API_BEGIN
   Ctx& c = x->c;
   if (!c.have_coef) return LMFHD_E_STATE;
-  d2d(c.io_a, xv, c.vlen * sizeof(double), c.s);
-  apply_matrix(c, c.io_a, b);
+  apply_matrix(c, apart(c, xv, b), b, Walls::any);
   return LMFHD_OK;
   API_END
 }
@@ -3939,8 +3958,7 @@ int lmfhd_apply_matrix_bc_dev(lmfhd_ctx* x, const double* xv, double* b, const d
   Ctx& c = x->c;
   if (!c.have_coef) return LMFHD_E_STATE;
   if (!xv || !b || !vel_bc_n || !vel_bc_t) { set_err("invalid argument"); return LMFHD_E_ARG; }
-  d2d(c.io_a, xv, c.vlen * sizeof(double), c.s);
-  apply_matrix(c, c.io_a, b);
+  apply_matrix(c, apart(c, xv, b), b, Walls::any);
   bc_lift(c, vel_bc_n, vel_bc_t, b, 1.0, -1.0);
   return LMFHD_OK;
   API_END
