@@ -899,26 +899,6 @@ static bool even_level(const Geo& g) {
   return true;
 }
 
-// The same functor over the components' item ranges in one flat launch, the components
-// alternating by workgroup (block b runs items 256 (b / DM) + [0, 256) of component b % DM): the
-// branch on the component is uniform in a workgroup
-template <class F, int DM>
-struct Comp3BlkFn {
-  F f[3];
-  unsigned n[3];
-  HD void operator()(long t) const {
-    const unsigned blk = (unsigned)(t >> 8), q = blk / DM;
-    const int a = (int)(blk - q * DM);
-    const unsigned u = (q << 8) + ((unsigned)t & 255u);
-    if (a == 0) {
-      if (u < n[0]) f[0](u);
-    } else if (DM == 2 || a == 1) {
-      if (u < n[1]) f[1](u);
-    } else if (u < n[2]) {
-      f[2](u);
-    }
-  }
-};
 // Levels a one-workgroup V-cycle takes (lmfhd_tune.coarse_n, mac_coarse_n = cn): those with every
 // extent <= cn and, from cn = 8 on, any level whose faces (cells) a workgroup of 1024 threads
 // holds in registers and whose work block fits LDS (|visc_type| 1: 3-D boxes up to about 12^3 in
@@ -1119,8 +1099,9 @@ struct StagMG {
 
   bool rows(const Geo& g) const { return rows_n > 0 && g.n[0] >= rows_n && !split_level(g); }
 
-  // one smoothing sweep set at level n
-  void smooth(hipStream_t s, int n, int nsweeps) {
+  // one smoothing sweep set at level n; skip: the first sweep's even parity is done already
+  // (stag_first; |visc_type| 1)
+  void smooth(hipStream_t s, int n, int nsweeps, bool skip = false) {
     Lev& l = L[n];
     const bool inplace = even_level(l.g);
     const bool by_rows = rows(l.g);
@@ -1159,7 +1140,7 @@ struct StagMG {
             F.ct = make_fastdiv((unsigned)ct);
             const int nw = w + ct * (dm == 3 ? l.g.n[2] : 1);
             F.omega = omega;
-            for (int par = 0; par < 2; ++par) {
+            for (int par = skip && m == 0 ? 1 : 0; par < 2; ++par) {
               F.par = par;
               launch_rows(s, nw, F);
             }
@@ -1193,7 +1174,7 @@ struct StagMG {
             for (int a = dm; a < 3; ++a) F.nc[a] = 0;
             F.ilv = cum >= GS_ILV_MIN ? 1 : 0;
             const long nl = F.ilv ? (long)dm * ((mx + 255) / 256) * 256 : cum;
-            for (int par = 0; par < 2; ++par) {
+            for (int par = skip && m == 0 ? 1 : 0; par < 2; ++par) {
               F.par = par;
               launch(s, nl, F);
             }
@@ -1212,7 +1193,7 @@ struct StagMG {
             F.dn = make_dec_color(l.g.n[0] + 1, l.g.n[1] + 1);
             F.Hn = pos3_half(l.g);
             F.mode = 0;
-            for (int par = 0; par < 2; ++par) {
+            for (int par = skip && m == 0 ? 1 : 0; par < 2; ++par) {
               F.par = par;
               launch(s, (long)F.Hn, F);
             }
@@ -1229,6 +1210,7 @@ struct StagMG {
         }
         for (int color = 1; color <= 2 * dm; ++color) {
           const int a = (color - 1) / 2, par = (color + 1) % 2;
+          if (skip && m == 0 && par == 0) continue;
           const int nx = fext(l.g, a, 0), ny = fext(l.g, a, 1);
           const long nc = (long)((nx + 1) / 2) * ny * fext(l.g, a, 2);
           if (inplace) {
@@ -1274,11 +1256,43 @@ struct StagMG {
     check_launch();
   }
 
-  // residual restriction, all components in one column launch; zeroes the coarse level's phi
-  template <int DM>
-  void restrict_res_dm(hipStream_t s, int n) {
+  int coarse_start_level() const { return smoother == 1 && coarse_l0 >= 0 ? std::min(coarse_l0, nl) : nl; }
+  // whether level n takes its first sweep's even parity from the kernel that forms its right-hand
+  // side: it is smoothed by launches of its own, from zero, with decoupled components
+  bool takes_first(int n) const {
+    return smoother == 1 && (vt == 1 || vt == -1) && n < coarse_start_level() && (n < nl - 1 ? nu_down : nu_bottom) > 0;
+  }
+  bool takes_first_level0() const { return max_vcycles == 1 && takes_first(0); }
+  // the residual of level n restricted to level n + 1, whose phi it sets
+  template <int VT, int DM>
+  void resid_restrict_vd(hipStream_t s, int n) {
     const Lev& f = L[n];
     Lev& c = L[n + 1];
+    if constexpr (VT == 1 || VT == -1) {
+      if (smoother == 1 && omega == T(1) && nu_down > 0 && even_level(f.g)) {
+        CompIlvFn<ResidRestrictFn<T, VT, DM>, DM> F;
+        ResidRestrictFn<T, VT, DM>& r = F.f;
+        r.gf = f.g;
+        r.gc = c.g;
+        r.C = f.C();
+        r.Cc = c.C();
+        r.omega = omega;
+        r.sf = f.sp;
+        r.sc = c.sp;
+        r.first = takes_first(n + 1);
+        for (int a = 0; a < 3; ++a) {
+          const int b = a < DM ? a : DM - 1;
+          r.phi[a] = f.phi[b];
+          r.rhs[a] = f.rhs[b];
+          r.rc[a] = c.rhs[b];
+          r.z[a] = c.phi[b];
+          r.dcc[a] = make_dec(fext(c.g, b, 0), fext(c.g, b, 1));
+        }
+        launch_comps<DM>(s, c.g, F);
+        return;
+      }
+    }
+    apply_all<T, VT, DM>(s, f.g, f.C(), f.phi, f.rhs, f.res, 1, rows(f.g), f.sp);
     AllFacesFn<RestrictFn<T, DM>, DM> F;
     F.g = c.g;
     for (int a = 0; a < 3; ++a) {
@@ -1289,10 +1303,23 @@ struct StagMG {
     F.cx = cs.cx;
     launch_cols(s, cs.ncols, cs.nz, cs.kc, F);
   }
-  void restrict_res(hipStream_t s, int n) {
-    if (dm == 3) restrict_res_dm<3>(s, n);
-    else restrict_res_dm<2>(s, n);
+  void resid_restrict(hipStream_t s, int n) {
+    dispatch_vd(vt, dm, [&](auto V, auto D) { resid_restrict_vd<decltype(V)::value, decltype(D)::value>(s, n); });
     check_launch();
+  }
+  // whether the launch above sets the first values (its two-step form zeroes)
+  bool first_done(int n) const {
+    return n > 0 && takes_first(n) && omega == T(1) && nu_down > 0 && even_level(L[n - 1].g);
+  }
+  // F over the faces of every component of geometry g
+  template <int DM, class F>
+  static void launch_comps(hipStream_t s, const Geo& g, CompIlvFn<F, DM>& f) {
+    long mx = 0;
+    for (int a = 0; a < 3; ++a) {
+      f.n[a] = a < DM ? (unsigned)fsize(g, a) : 0u;
+      mx = std::max(mx, (long)f.n[a]);
+    }
+    launch(s, (long)DM * ((mx + 255) / 256) * 256, f);
   }
   // prolongation-add into level n from the coarse side (ProlongCFn), all components in one
   // launch
@@ -1305,15 +1332,18 @@ struct StagMG {
   }
   template <int DM>
   void prolong_all(hipStream_t s, Lev& f, const Lev& c) {
-    Comp3BlkFn<ProlongCFn<T, DM>, DM> F;
-    long mx = 0;
+    CompIlvFn<ProlongCFn<T, DM>, DM> F;
+    F.f.gf = f.g;
+    F.f.gc = c.g;
+    F.f.sf = f.sp;
+    F.f.sc = c.sp;
     for (int a = 0; a < 3; ++a) {
       const int b = a < DM ? a : DM - 1;
-      F.f[a] = ProlongCFn<T, DM>{f.g, c.g, f.phi[b], c.phi[b], b, make_dec(fext(c.g, b, 0), fext(c.g, b, 1)), f.sp, c.sp};
-      F.n[a] = a < DM ? (unsigned)fsize(c.g, b) : 0u;
-      mx = std::max(mx, (long)F.n[a]);
+      F.f.fs[a] = f.phi[b];
+      F.f.cs[a] = c.phi[b];
+      F.f.dcc[a] = make_dec(fext(c.g, b, 0), fext(c.g, b, 1));
     }
-    launch(s, (long)DM * ((mx + 255) / 256) * 256, F);
+    launch_comps<DM>(s, c.g, F);
   }
 
   // levels l0..nl-1 of one V-cycle in one workgroup (coarse.h); phi of level l0 > 0 arrives zeroed
@@ -1378,8 +1408,9 @@ struct StagMG {
     check_launch();
   }
 
-  // V-cycles on L[0].rhs with L[0].phi as the initial guess (stag_mg_solver.f90:323-807)
-  void solve(hipStream_t s, Reducer& R) {
+  // V-cycles on L[0].rhs with L[0].phi as the initial guess (stag_mg_solver.f90:323-807); first: phi
+  // was zero and holds its first sweep's even parity (takes_first_level0)
+  void solve(hipStream_t s, Reducer& R, bool first = false) {
     double resid0[3] = {0, 0, 0};
     if (max_vcycles > 1) {
       residual(s, 0);
@@ -1396,19 +1427,18 @@ struct StagMG {
       if (allzero) return;
       if (anyzero) for (int a = 0; a < dm; ++a) resid0[a] = mx;
     }
-    const int l0 = (smoother == 1) ? coarse_l0 : nl;
+    const int l0 = coarse_start_level();
     for (int vc = 0; vc < max_vcycles; ++vc) {
-      // the restriction into level n + 1 zeroes that level's phi (every face; the slack slots of
+      // the restriction into level n + 1 sets that level's phi (every face; the slack slots of
       // split storage are zero from allocation and never written)
       for (int n = 0; n < std::min(l0, nl - 1); ++n) {
-        smooth(s, n, nu_down);
-        residual(s, n);
-        restrict_res(s, n);
+        smooth(s, n, nu_down, n == 0 ? first : first_done(n));
+        resid_restrict(s, n);
       }
       if (l0 < nl) {
         coarse(s);
       } else {
-        smooth(s, nl - 1, nu_bottom);
+        smooth(s, nl - 1, nu_bottom, nl == 1 ? first : first_done(nl - 1));
       }
       for (int n = std::min(l0, nl - 1) - 1; n >= 0; --n) {
         prolong(s, n);
@@ -1515,13 +1545,15 @@ struct MacMG {
     }
     check_launch();
   }
+  // sweeps of level n; skip: the first sweep's even parity is done already (mac_first)
   template <int DM>
-  void gs(hipStream_t s, int n, int nsweeps) {
+  void gs(hipStream_t s, int n, int nsweeps, bool skip = false) {
     Lev& l = L[n];
     const long nc = (long)((l.g.n[0] + 1) / 2) * l.g.n[1] * l.g.n[2];
     const bool inplace = even_level(l.g);
     for (int m = 0; m < nsweeps; ++m)
       for (int par = 0; par < 2; ++par) {
+        if (skip && m == 0 && par == 0) continue;
         if (inplace) {
           launch(s, nc, MacGsFn<T, DM>{l.g, {l.b[0], l.b[1], l.b[2]}, l.h2i, l.phi, l.rhs, par, make_dec_color(l.g.n[0], l.g.n[1])});
         } else {
@@ -1529,6 +1561,42 @@ struct MacMG {
           launch(s, nc, CopyColorCellFn<T>{l.g, l.phi, l.tmp, par, make_dec_color(l.g.n[0], l.g.n[1])});
         }
       }
+  }
+  // whether level n takes its first sweep's even parity from the kernel that forms its rhs: it is
+  // smoothed from zero by launches of its own
+  bool takes_first(int n) const {
+    return n < coarse_start_level() && (n < nl - 1 ? nu_down : nu_bottom) > 0 && max_vcycles > 0;
+  }
+  int coarse_start_level() const { return coarse_l0 < 0 ? nl : std::min(coarse_l0, nl); }
+  // the residual of level n restricted to level n + 1
+  template <int DM>
+  void restrict_res(hipStream_t s, int n) {
+    const Lev& f = L[n];
+    Lev& c = L[n + 1];
+    MacResidRestrictFn<T, DM> F{f.g, c.g, {f.b[0], f.b[1], f.b[2]}, f.h2i, f.phi, f.rhs, c.rhs, make_dec(c.g.n[0], c.g.n[1]), c.phi};
+    for (int d = 0; d < 3; ++d) F.bc[d] = c.b[d];
+    F.h2ic = c.h2i;
+    F.half = nu_down > 0 && even_level(f.g);
+    // the bottom's rhs has its mean removed before it is smoothed
+    F.first = n + 1 < nl - 1 && takes_first(n + 1);
+    launch(s, csize(c.g), F);
+  }
+  // the prolongation from level n + 1 added to level n, then nu_up sweeps: in one with the first of
+  // them where that runs in place
+  template <int DM>
+  void prolong_gs(hipStream_t s, int n) {
+    Lev& f = L[n];
+    const Lev& c = L[n + 1];
+    if (nu_up > 0 && even_level(f.g)) {
+      const long nc = (long)(f.g.n[0] / 2) * f.g.n[1] * f.g.n[2];
+      const Dec dc = make_dec_color(f.g.n[0], f.g.n[1]);
+      launch(s, nc, MacGsUpFn<T, DM, 0>{f.g, c.g, {f.b[0], f.b[1], f.b[2]}, f.h2i, f.phi, f.rhs, c.phi, dc});
+      launch(s, nc, MacGsUpFn<T, DM, 1>{f.g, c.g, {f.b[0], f.b[1], f.b[2]}, f.h2i, f.phi, f.rhs, c.phi, dc});
+      gs<DM>(s, n, nu_up - 1);
+      return;
+    }
+    launch(s, csize(f.g), MacProlongFn<T>{f.g, c.g, f.phi, c.phi, make_dec(f.g.n[0], f.g.n[1])});
+    gs<DM>(s, n, nu_up);
   }
   MacCoarseArgs<T>* coarse_args = nullptr;
   int coarse_l0 = -1;
@@ -1574,47 +1642,34 @@ struct MacMG {
     launch_mac_coarse<T>(s, dm, coarse_nt, coarse_form, coarse_args);
     check_launch();
   }
+  // first: level 0's phi holds its first sweep's even parity (the first V-cycle only)
   template <int DM>
-  void solve_dm(hipStream_t s) {
-    const int l0 = coarse_l0;
-    if (l0 < nl) {
-      for (int vc = 0; vc < max_vcycles; ++vc) {
-        for (int n = 0; n < l0; ++n) {  // the restriction zeroes phi of level n + 1
-          gs<DM>(s, n, nu_down);
-          const Lev& f = L[n];
-          Lev& c = L[n + 1];
-          launch(s, csize(c.g), MacResidRestrictFn<T, DM>{f.g, c.g, {f.b[0], f.b[1], f.b[2]}, f.h2i, f.phi, f.rhs, c.rhs, make_dec(c.g.n[0], c.g.n[1]), c.phi});
-        }
-        coarse(s);
-        for (int n = l0 - 1; n >= 0; --n) {
-          launch(s, csize(L[n].g), MacProlongFn<T>{L[n].g, L[n + 1].g, L[n].phi, L[n + 1].phi, make_dec(L[n].g.n[0], L[n].g.n[1])});
-          gs<DM>(s, n, nu_up);
-        }
-      }
-      check_launch();
-      return;
-    }
+  void solve_dm(hipStream_t s, bool first) {
+    const int l0 = coarse_start_level();
     for (int vc = 0; vc < max_vcycles; ++vc) {
-      for (int n = 0; n < nl - 1; ++n) {  // the restriction zeroes phi of level n + 1
-        gs<DM>(s, n, nu_down);
-        const Lev& f = L[n];
-        Lev& c = L[n + 1];
-        launch(s, csize(c.g), MacResidRestrictFn<T, DM>{f.g, c.g, {f.b[0], f.b[1], f.b[2]}, f.h2i, f.phi, f.rhs, c.rhs, make_dec(c.g.n[0], c.g.n[1]), c.phi});
+      auto done = [&](int n) { return n == 0 ? first && vc == 0 : n < nl - 1 && takes_first(n); };
+      for (int n = 0; n < std::min(l0, nl - 1); ++n) {  // the restriction sets phi of level n + 1
+        gs<DM>(s, n, nu_down, done(n));
+        restrict_res<DM>(s, n);
       }
-      remove_mean_small<T>(s, L[nl - 1].rhs, csize(L[nl - 1].g));
-      gs<DM>(s, nl - 1, nu_bottom);
-      for (int n = nl - 2; n >= 0; --n) {
-        launch(s, csize(L[n].g), MacProlongFn<T>{L[n].g, L[n + 1].g, L[n].phi, L[n + 1].phi, make_dec(L[n].g.n[0], L[n].g.n[1])});
-        gs<DM>(s, n, nu_up);
+      if (l0 < nl) {
+        coarse(s);
+      } else {
+        remove_mean_small<T>(s, L[nl - 1].rhs, csize(L[nl - 1].g));
+        gs<DM>(s, nl - 1, nu_bottom);
       }
+      for (int n = std::min(l0, nl - 1) - 1; n >= 0; --n) prolong_gs<DM>(s, n);
     }
     check_launch();
   }
-  // phi (level 0) from zero for L[0].rhs; phi_zeroed: the caller's last kernel zeroed it
-  void solve(hipStream_t s, bool phi_zeroed = false) {
-    if (!phi_zeroed) fill<T>(s, L[0].phi, csize(L[0].g), T(0));
-    if (dm == 3) solve_dm<3>(s);
-    else solve_dm<2>(s);
+  // phi (level 0) from zero for L[0].rhs.  The caller's last kernel has set phi: 0 nothing yet,
+  // 1 to zero, 2 to its first sweep's even parity (takes_first_level0)
+  enum class Phi { unset, zero, first };
+  bool takes_first_level0() const { return nl > 1 && takes_first(0); }
+  void solve(hipStream_t s, Phi phi = Phi::unset) {
+    if (phi == Phi::unset) fill<T>(s, L[0].phi, csize(L[0].g), T(0));
+    if (dm == 3) solve_dm<3>(s, phi == Phi::first);
+    else solve_dm<2>(s, phi == Phi::first);
   }
 };
 
@@ -2007,36 +2062,42 @@ static void precon(Ctx& c, StagMG<T>& mg, MacMG<T>& mac, T* macrhs, const double
   const int dm = c.dm;
   auto& l0 = mg.L[0];
   const ColShape cs = col_shape(c.g);
-  auto enter = [&](auto D) {
-    constexpr int DM = decltype(D)::value;
-    AllFacesFn<EnterFn<T>, DM> F;
+  const bool first = mg.takes_first_level0();
+  dispatch_vd(c.d.visc_type, dm, [&](auto V, auto D) {
+    constexpr int VT = decltype(V)::value, DM = decltype(D)::value;
+    AllFacesFn<EnterFn<T, VT, DM>, DM> F;
     F.g = c.g;
     for (int a = 0; a < 3; ++a) {
       const int q = a < DM ? a : DM - 1;
-      F.f[a] = EnterFn<T>{b + c.off[q], l0.rhs[q], l0.phi[q], l0.g, q, l0.sp};
+      F.f[a] = EnterFn<T, VT, DM>{b + c.off[q], l0.rhs[q], l0.phi[q], l0.g, l0.C(), mg.omega, l0.sp, first ? 1 : 0};
     }
     F.cx = cs.cx;
     launch_cols(s, cs.ncols, cs.nz, cs.kc, F);
-  };
-  if (dm == 3) enter(std::integral_constant<int, 3>{});
-  else enter(std::integral_constant<int, 2>{});
-  mg.solve(s, c.R);
+  });
+  mg.solve(s, c.R, first);
   // mac_rhs = D x_u + b_p (kept twice: the MAC solve consumes its copy)
+  const int mac_first = mac.takes_first_level0();
   const T* ph[3] = {l0.phi[0], l0.phi[1], dm == 3 ? l0.phi[2] : l0.phi[1]};
   if (dm == 3) {
     DivPlusFn<T, 3> f{c.g, {ph[0], ph[1], ph[2]}, b + c.off[3], mac.L[0].rhs, T(1.0 / c.dx), make_dec(c.g.n[0], c.g.n[1])};
     f.out2 = macrhs;
     f.sp = l0.sp;
     f.z = mac.L[0].phi;
+    f.first = mac_first;
+    for (int d = 0; d < 3; ++d) f.b[d] = mac.L[0].b[d];
+    f.h2i = mac.L[0].h2i;
     launch(s, c.nc, f);
   } else {
     DivPlusFn<T, 2> f{c.g, {ph[0], ph[1], ph[2]}, b + c.off[3], mac.L[0].rhs, T(1.0 / c.dx), make_dec(c.g.n[0], c.g.n[1])};
     f.out2 = macrhs;
     f.sp = l0.sp;
     f.z = mac.L[0].phi;
+    f.first = mac_first;
+    for (int d = 0; d < 3; ++d) f.b[d] = mac.L[0].b[d];
+    f.h2i = mac.L[0].h2i;
     launch(s, c.nc, f);
   }
-  mac.solve(s, true);
+  mac.solve(s, mac_first ? MacMG<T>::Phi::first : MacMG<T>::Phi::zero);
   auto leave = [&](auto D) {
     constexpr int DM = decltype(D)::value;
     FacesCellFn<PreconFaceFn<T>, PreconCellFn<T>, DM> F;
@@ -2135,7 +2196,7 @@ static void precon_general(Ctx& c, StagMG<T>& mg, MacMG<T>& mac, T* macrhs, cons
   if (apt == 1) {  // -1
     stag_solve(true, nullptr);
     div_plus_bp();
-    mac.solve(s, true);
+    mac.solve(s, MacMG<T>::Phi::zero);
     for (int a = 0; a < dm; ++a)
       launch(s, c.nf[a], PreconFaceFn<T>{c.g, l0.phi[a], m0.phi, c.alpha64[a], x + c.off[a], dxinv, a,
                                           make_dec(fext(c.g, a, 0), fext(c.g, a, 1)), l0.sp});
@@ -2151,7 +2212,7 @@ static void precon_general(Ctx& c, StagMG<T>& mg, MacMG<T>& mac, T* macrhs, cons
   } else if (apt == 2 || apt == 5) {  // lower triangular (:196-276)
     stag_solve(true, nullptr);
     div_plus_bp();
-    if (mac_solve) mac.solve(s, true);
+    if (mac_solve) mac.solve(s, MacMG<T>::Phi::zero);
     if (mmu) visc_schur<T>(c, mg, mac, *mmu, macrhs, mac_solve, xp);
     else schur_simple(macrhs);
     if (pt == -2 || pt == -5) launch(s, c.nc, ConvertFn<double, double>{xp, xp, -1.0});

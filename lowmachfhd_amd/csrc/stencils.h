@@ -277,9 +277,9 @@ HD T lphi(const Geo& g, const Coefs<T>& C, T* const* phi, int a, int i, int j, i
 
 // diagonal coefficient only (stag_mg_update "fac")
 template <typename T, int VT, int DM>
-HD T diag_at(const Geo& g, const Coefs<T>& C, int a, int i, int j, int k) {
+HD T diag_at(const Geo& g, const Coefs<T>& C, int a, int i, int j, int k, int sp = 0) {
   const int ea0 = a == 0, ea1 = a == 1, ea2 = a == 2;
-  const T alpha = ld(C.alpha[a], (unsigned)fidx(g, a, i, j, k)) * C.theta;
+  const T alpha = ld(C.alpha[a], lidx(g, a, i, j, k, sp)) * C.theta;
   if constexpr (VT > 0) {
     const T b0 = C.beta[0];
     if constexpr (VT == 1) return alpha + T(2 * DM) * b0 * C.dxsqinv;
@@ -757,7 +757,7 @@ struct RestrictFn {
       if (z) st(z, o, T(0));
     });
   }
-  HD void put(int i, int j, int k, long t, T v) const {
+  HD void put(int i, int j, int k, long t, const int, T v) const {
     const unsigned o = sc ? sidx(gc, a, i, j, k) : (unsigned)t;
     st(c, o, v);
     if (z) st(z, o, T(0));
@@ -786,6 +786,105 @@ struct RestrictFn {
   }
 };
 
+// The first value a Gauss-Seidel sweep from phi = 0 gives face (i,j,k) of component a (|visc_type|
+// 1): omega r / diag on the even parity (L phi = 0 there), 0 on the odd one, which the sweep's
+// second step takes from 0.  Written by the kernel that forms the level's right-hand side r, it
+// saves the sweep's first step a launch and a pass.
+template <typename T, int VT, int DM>
+HD T stag_first(const Geo& g, const Coefs<T>& C, T omega, T r, int a, int i, int j, int k, int sp) {
+  const int I[3] = {i, j, k};
+  const T d = diag_at<T, VT, DM>(g, C, a, i, j, k, sp);
+  return ((i + j + k) & 1) == 0 && !wall_face(g, a, I[a]) ? omega * r / d : T(0);
+}
+// A functor's items for every component in one flat launch, the components alternating by
+// workgroup: block b runs items 256 (b / DM) + [0, 256) of component b % DM through f.at(item,
+// component), the component a literal
+template <class F, int DM>
+struct CompIlvFn {
+  F f;
+  unsigned n[3];
+  HD void operator()(long t) const {
+    const unsigned blk = (unsigned)(t >> 8), q = blk / DM;
+    const int a = (int)(blk - q * DM);
+    const unsigned u = (q << 8) + ((unsigned)t & 255u);
+    by_comp<DM>(a, [&](const int ac) __attribute__((always_inline)) {
+      if (u < n[ac]) f.at(u, ac);
+    });
+  }
+};
+// The residual of a level restricted to the next (RestrictFn's 12 points) without a residual array,
+// for a level just smoothed in place on its odd parity with omega = 1 and |visc_type| 1: the odd
+// faces' residuals are then zero up to rounding (the step solved their equations, and nothing they
+// read has changed since), so of a coarse face's twelve fine faces the six even ones are formed
+// and summed.  Beside a wall across a, a face reads its own reflection, which did change: there
+// the odd ones are formed too.  A launch and the array's write and twelvefold read saved against residual then
+// restriction.  first: the coarse phi gets stag_first, else zero.
+template <typename T, int VT, int DM>
+struct ResidRestrictFn {
+  Geo gf, gc;
+  Coefs<T> C, Cc;
+  T* phi[3];
+  const T* rhs[3];
+  T* rc[3];
+  T* z[3];
+  Dec dcc[3];
+  T omega;
+  int sf, sc, first;
+  HD void at(unsigned t, const int a) const {
+    int i, j, k;
+    decode3(t, dcc[a], i, j, k);
+    const int I[3] = {i, j, k};
+    int tb[2];
+    transverse(a, tb[0], tb[1]);
+    T s0 = T(0), sp = T(0), sm = T(0);
+    auto resid = [&](int d, int q) {  // fine face 2 I + d along a, offset bits q across it
+      int F[3] = {2 * i, 2 * j, DM == 3 ? 2 * k : 0};
+      F[tb[0]] += q & 1;
+      if (DM == 3) F[tb[1]] += q >> 1;
+      const int v = F[a] + d, n = gf.n[a];
+      F[a] = v < 0 ? v + n : (v > n ? v - n : v);
+      const T r = ld(rhs[a], lidx(gf, a, F[0], F[1], F[2], sf));
+      return r - lphi<T, VT, DM>(gf, C, phi, a, F[0], F[1], F[2], nullptr, nullptr, sf);
+    };
+#pragma unroll
+    for (int q = 0; q < (1 << (DM - 1)); ++q) {
+      const bool odd = ((q ^ (q >> 1)) & 1) != 0;  // the parity of the offsets across
+      if (!odd) s0 += resid(0, q);
+      else {
+        sp += resid(1, q);
+        sm += resid(-1, q);
+      }
+    }
+    bool beside = false;
+#pragma unroll
+    for (int t = 0; t < DM - 1; ++t) beside = beside || (!gc.per[tb[t]] && (I[tb[t]] == 0 || I[tb[t]] == gc.n[tb[t]] - 1));
+    if (beside) {
+#pragma unroll 1
+      for (int e = 0; e < 3 << (DM - 1); ++e) {
+        const int q = e & ((1 << (DM - 1)) - 1), w = e >> (DM - 1);  // w: 0 on the face, 1 above, 2 below
+        if (((q ^ (q >> 1)) & 1) == (w ? 1 : 0)) continue;            // formed above
+        bool at_wall = false;
+#pragma unroll
+        for (int t = 0; t < DM - 1; ++t) {
+          const int v = 2 * I[tb[t]] + ((q >> t) & 1);
+          at_wall = at_wall || (!gf.per[tb[t]] && (v == 0 || v == gf.n[tb[t]] - 1));
+        }
+        if (!at_wall) continue;
+        const T x = resid(w == 0 ? 0 : (w == 1 ? 1 : -1), q);
+        if (w == 0) s0 += x;
+        else if (w == 1) sp += x;
+        else sm += x;
+      }
+    }
+    T r = DM == 3 ? T(0.125) * s0 + T(0.0625) * sp + T(0.0625) * sm : T(0.25) * s0 + T(0.125) * (sp + sm);
+    if (wall_face(gc, a, I[a])) r = T(0);
+    const unsigned o = sc ? sidx(gc, a, i, j, k) : t;
+    const T f = first ? stag_first<T, VT, DM>(gc, Cc, omega, r, a, i, j, k, sc) : T(0);
+    st(rc[a], o, r);
+    st(z[a], o, f);
+  }
+};
+
 // Prolongation-add (stag_mg_solver.f90:1365-1628) from the coarse side: one thread per coarse
 // face (I,J,K) of component a adds to the 2^dm fine faces (2I, 2J+dj, 2K+dk) and, below the last coarse face along a, to the
 // 2^dm faces (2I+1, ...) between I and I+1.  Those fine faces use the coarse values at I, I+1
@@ -794,70 +893,69 @@ struct RestrictFn {
 template <typename T, int DM>
 struct ProlongCFn {
   Geo gf, gc;
-  T* f;
-  const T* c;
-  int a;
-  Dec dcc;             // decoder of the coarse face array of component a
+  T* fs[3];
+  const T* cs[3];
+  Dec dcc[3];          // decoders of the coarse face arrays
   int sf = 0, sc = 0;  // fine / coarse arrays in parity-split storage
-  HD void operator()(long t) const {
+  HD void at(unsigned t, const int ac) const {
     int I0, J0, K0;
-    decode3(t, dcc, I0, J0, K0);
-    by_comp<DM>(a, [&](const int ac) __attribute__((always_inline)) {
-      int tb[2];
-      transverse(ac, tb[0], tb[1]);
-      const int C0[3] = {I0, J0, K0};
-      constexpr int NK = DM == 3 ? 3 : 1;
-      T P[2][3][NK];
+    decode3(t, dcc[ac], I0, J0, K0);
+    T* const f = fs[ac];
+    const T* const c = cs[ac];
+    int tb[2];
+    transverse(ac, tb[0], tb[1]);
+    const int C0[3] = {I0, J0, K0};
+    constexpr int NK = DM == 3 ? 3 : 1;
+    T P[2][3][NK];
 #pragma unroll
-      for (int na = 0; na < 2; ++na)
+    for (int na = 0; na < 2; ++na)
 #pragma unroll
-        for (int m = 0; m < 3; ++m)
+      for (int m = 0; m < 3; ++m)
 #pragma unroll
-          for (int n = 0; n < NK; ++n) {
-            int J[3] = {C0[0], C0[1], C0[2]};
-            J[ac] += na;
-            J[tb[0]] += m - 1;
-            if (DM == 3) J[tb[1]] += n - 1;
-            P[na][m][n] = vel_at(c, gc, ac, J[0], J[1], J[2], (const T*)nullptr, sc);
+        for (int n = 0; n < NK; ++n) {
+          int J[3] = {C0[0], C0[1], C0[2]};
+          J[ac] += na;
+          J[tb[0]] += m - 1;
+          if (DM == 3) J[tb[1]] += n - 1;
+          P[na][m][n] = vel_at(c, gc, ac, J[0], J[1], J[2], (const T*)nullptr, sc);
+        }
+    const int last = C0[ac] == fext(gc, ac, ac) - 1;  // no fine face beyond the last coarse one
+#pragma unroll
+    for (int fa = 0; fa < 2; ++fa) {
+      if (fa == 1 && last) continue;
+#pragma unroll
+      for (int d0 = 0; d0 < 2; ++d0)
+#pragma unroll
+        for (int d1 = 0; d1 < (DM == 3 ? 2 : 1); ++d1) {
+          int F[3] = {2 * C0[0], 2 * C0[1], 2 * C0[2]};
+          F[ac] += fa;
+          F[tb[0]] += d0;
+          if (DM == 3) F[tb[1]] += d1;
+          const unsigned o = lidx(gf, ac, F[0], F[1], F[2], sf);
+          const T old = ld(f, o);
+          const int m = d0 == 0 ? 0 : 2, n = DM == 3 ? (d1 == 0 ? 0 : 2) : 0, n1 = DM == 3 ? 1 : 0;
+          T add;
+          if (DM == 3) {
+            const T p000 = P[0][1][n1], p0b0 = P[0][m][n1], p00c = P[0][1][n], p0bc = P[0][m][n];
+            const T p100 = P[1][1][n1], p1b0 = P[1][m][n1], p10c = P[1][1][n], p1bc = P[1][m][n];
+            const T se = T(9.0 / 16.0) * p000 + T(3.0 / 16.0) * p0b0 + T(3.0 / 16.0) * p00c + T(1.0 / 16.0) * p0bc;
+            const T so = T(9.0 / 32.0) * p000 + T(3.0 / 32.0) * p0b0 + T(3.0 / 32.0) * p00c + T(1.0 / 32.0) * p0bc +
+                         T(9.0 / 32.0) * p100 + T(3.0 / 32.0) * p1b0 + T(3.0 / 32.0) * p10c + T(1.0 / 32.0) * p1bc;
+            add = fa == 0 ? se : so;
+          } else {
+            const T p000 = P[0][1][0], p0b0 = P[0][m][0], p100 = P[1][1][0], p1b0 = P[1][m][0];
+            const T se = T(0.75) * p000 + T(0.25) * p0b0;
+            const T so = T(0.375) * p000 + T(0.125) * p0b0 + T(0.375) * p100 + T(0.125) * p1b0;
+            add = fa == 0 ? se : so;
           }
-      const int last = C0[ac] == fext(gc, ac, ac) - 1;  // no fine face beyond the last coarse one
-#pragma unroll
-      for (int fa = 0; fa < 2; ++fa) {
-        if (fa == 1 && last) continue;
-#pragma unroll
-        for (int d0 = 0; d0 < 2; ++d0)
-#pragma unroll
-          for (int d1 = 0; d1 < (DM == 3 ? 2 : 1); ++d1) {
-            int F[3] = {2 * C0[0], 2 * C0[1], 2 * C0[2]};
-            F[ac] += fa;
-            F[tb[0]] += d0;
-            if (DM == 3) F[tb[1]] += d1;
-            const unsigned o = lidx(gf, ac, F[0], F[1], F[2], sf);
-            const T old = ld(f, o);
-            const int m = d0 == 0 ? 0 : 2, n = DM == 3 ? (d1 == 0 ? 0 : 2) : 0, n1 = DM == 3 ? 1 : 0;
-            T add;
-            if (DM == 3) {
-              const T p000 = P[0][1][n1], p0b0 = P[0][m][n1], p00c = P[0][1][n], p0bc = P[0][m][n];
-              const T p100 = P[1][1][n1], p1b0 = P[1][m][n1], p10c = P[1][1][n], p1bc = P[1][m][n];
-              const T se = T(9.0 / 16.0) * p000 + T(3.0 / 16.0) * p0b0 + T(3.0 / 16.0) * p00c + T(1.0 / 16.0) * p0bc;
-              const T so = T(9.0 / 32.0) * p000 + T(3.0 / 32.0) * p0b0 + T(3.0 / 32.0) * p00c + T(1.0 / 32.0) * p0bc +
-                           T(9.0 / 32.0) * p100 + T(3.0 / 32.0) * p1b0 + T(3.0 / 32.0) * p10c + T(1.0 / 32.0) * p1bc;
-              add = fa == 0 ? se : so;
-            } else {
-              const T p000 = P[0][1][0], p0b0 = P[0][m][0], p100 = P[1][1][0], p1b0 = P[1][m][0];
-              const T se = T(0.75) * p000 + T(0.25) * p0b0;
-              const T so = T(0.375) * p000 + T(0.125) * p0b0 + T(0.375) * p100 + T(0.125) * p1b0;
-              add = fa == 0 ? se : so;
-            }
-            st(f, o, wall_face(gf, ac, F[ac]) ? old : old + add);
-          }
-      }
-    });
+          st(f, o, wall_face(gf, ac, F[ac]) ? old : old + add);
+        }
+    }
   }
 };
 
 // every component of a per-face functor F (with eval(i, j, k, offset, component) -> value and
-// put(offset, value)) in one column launch
+// put(i, j, k, offset, component, value)) in one column launch
 // over the nodal box of geometry g
 template <class F, int DM>
 struct AllFacesFn {
@@ -881,7 +979,7 @@ struct AllFacesFn {
       }
 #pragma unroll
       for (int a = 0; a < DM; ++a)
-        if (face_in(g, a, i, j, k)) f[a].put(i, j, k, o[a], v[a]);
+        if (face_in(g, a, i, j, k)) f[a].put(i, j, k, o[a], a, v[a]);
     }
   }
 };
@@ -905,22 +1003,28 @@ struct FacesCellFn {
   }
 };
 
-// multigrid entry: rhs = b (converted), phi = 0; with sp the level's arrays are in
-// parity-split storage of geometry g, component a
-template <typename T>
+// multigrid entry of component a: rhs = b (converted), phi = 0 or (first) stag_first; with sp the
+// level's arrays are in parity-split storage of geometry g
+template <typename T, int VT, int DM>
 struct EnterFn {
-  using value_type = T;
+  struct value_type {
+    T r, f;
+  };
   const double* b;
   T* rhs;
   T* phi;
   Geo g{};
-  int a = 0;
-  int sp = 0;
-  HD T eval(int, int, int, long t, int) const { return T(b[t]); }
-  HD void put(int i, int j, int k, long t, T v) const {
+  Coefs<T> C{};
+  T omega = T(0);
+  int sp = 0, first = 0;
+  HD value_type eval(int i, int j, int k, long t, const int a) const {
+    const T r = T(b[t]);
+    return {r, first ? stag_first<T, VT, DM>(g, C, omega, r, a, i, j, k, sp) : T(0)};
+  }
+  HD void put(int i, int j, int k, long t, const int a, value_type v) const {
     const unsigned m = sp ? sidx(g, a, i, j, k) : (unsigned)t;
-    rhs[m] = v;
-    phi[m] = T(0);
+    rhs[m] = v.r;
+    phi[m] = v.f;
   }
 };
 
@@ -1002,6 +1106,67 @@ struct MacGsFn {  // in place, one parity (consistent red-black colouring)
   }
 };
 
+// the first value a Gauss-Seidel sweep from phi = 0 gives cell (i,j,k): rhs / diag on the even parity
+// (L phi = 0 there), 0 on the odd one, which the sweep's second step takes from 0.  Written by the
+// kernel that forms the level's rhs, it saves the sweep's first step a launch and a pass.
+template <typename T, int DM>
+HD T mac_first(const Geo& g, T* const* b, T h2i, T rhs, int i, int j, int k) {
+  T dsum = T(0);
+#pragma unroll
+  for (int d = 0; d < DM; ++d)
+    dsum += ld(b[d], (unsigned)fidx(g, d, i + (d == 0), j + (d == 1), k + (d == 2))) + ld(b[d], (unsigned)fidx(g, d, i, j, k));
+  const T diag = -dsum * h2i;
+  return ((i + j + k) & 1) == 0 && diag != T(0) ? rhs / diag : T(0);
+}
+// One parity of the sweep after a prolongation that has not been added yet: PASS 0 reads phi + the
+// parent's value everywhere, PASS 1 (the neighbours are done) for the cell itself only
+template <typename T, int DM, int PASS>
+struct MacGsUpFn {
+  Geo g, gc;
+  T* b[3];
+  T h2i;
+  T* phi;
+  const T* rhs;
+  const T* c;  // the coarse level's phi
+  Dec dc;
+  HD T at(int i, int j, int k) const {
+    int I[3] = {i, j, k};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {  // cc_at's rules
+      const int n = g.n[d], v = I[d];
+      const bool lo = v < 0, hi = v >= n;
+      const int vp = v + (lo ? n : 0) - (hi ? n : 0);
+      const int vw = lo ? 0 : (hi ? n - 1 : v);
+      I[d] = vw + g.per[d] * (vp - vw);
+    }
+    const T p = ld(phi, (unsigned)cidx(g, I[0], I[1], I[2]));
+    return p + ld(c, (unsigned)cidx(gc, I[0] >> 1, I[1] >> 1, DM == 3 ? I[2] >> 1 : 0));
+  }
+  HD void operator()(long t) const {
+    int i, j, k;
+    if (!decode_color(t, dc, PASS, i, j, k)) return;
+    const unsigned o = (unsigned)cidx(g, i, j, k);
+    const T old = ld(phi, o) + ld(c, (unsigned)cidx(gc, i >> 1, j >> 1, DM == 3 ? k >> 1 : 0));
+    const T r = ld(rhs, o);
+    T s = T(0), dsum = T(0);
+#pragma unroll
+    for (int d = 0; d < DM; ++d) {  // mac_L's sums
+      const int e0 = d == 0, e1 = d == 1, e2 = d == 2;
+      const T bp = ld(b[d], (unsigned)fidx(g, d, i + e0, j + e1, k + e2));
+      const T bm = ld(b[d], (unsigned)fidx(g, d, i, j, k));
+      const T pp = PASS == 0 ? at(i + e0, j + e1, k + e2) : cc_at(phi, g, i + e0, j + e1, k + e2);
+      const T pm = PASS == 0 ? at(i - e0, j - e1, k - e2) : cc_at(phi, g, i - e0, j - e1, k - e2);
+      // a neighbour beyond a wall is the cell itself, which this step has not written yet
+      const T ap = PASS == 1 && !g.per[d] && (d == 0 ? i : (d == 1 ? j : k)) == g.n[d] - 1 ? old : pp;
+      const T am = PASS == 1 && !g.per[d] && (d == 0 ? i : (d == 1 ? j : k)) == 0 ? old : pm;
+      s += bp * (ap - old) - bm * (old - am);
+      dsum += bp + bm;
+    }
+    const T L = s * h2i, diag = -dsum * h2i;
+    st(phi, o, diag != T(0) ? old + (r - L) / diag : old);
+  }
+};
+
 template <typename T, int DM>
 struct MacGsNewFn {  // phase 1 of the two-phase sweep: new values of one parity into tmp
   Geo g;
@@ -1037,8 +1202,12 @@ struct CopyColorCellFn {  // phase 2: phi <- tmp on one parity
   }
 };
 
+// Coarse rhs = mean of the children's residuals.  half: the level was last smoothed on its odd
+// parity, in place, so the odd children's residuals are zero up to rounding (the step solved
+// their equations and nothing they read has changed since); only the even four are formed.
+// first: the coarse phi gets its first sweep's even parity (mac_first), else zero.
 template <typename T, int DM>
-struct MacResidRestrictFn {  // coarse rhs = mean of the children's residuals
+struct MacResidRestrictFn {
   Geo gf, gc;
   T* b[3];
   T h2i;
@@ -1046,18 +1215,24 @@ struct MacResidRestrictFn {  // coarse rhs = mean of the children's residuals
   const T* rhs;
   T* rc;
   Dec dc;
-  T* z = nullptr;  // when set, the coarse level's phi, zeroed
+  T* z;      // the coarse level's phi
+  T* bc[3];  // the coarse level's coefficients
+  T h2ic;
+  int half, first;
   HD void operator()(long t) const {
     int i, j, k;
     decode3(t, dc, i, j, k);
     T s = T(0);
 #pragma unroll
     for (int q = 0; q < (1 << DM); ++q) {
+      const int odd = (q ^ (q >> 1) ^ (q >> 2)) & 1;
+      if (half && odd) continue;
       const int ii = 2 * i + (q & 1), jj = 2 * j + ((q >> 1) & 1), kk = DM == 3 ? 2 * k + ((q >> 2) & 1) : 0;
-      s += rhs[cidx(gf, ii, jj, kk)] - mac_L<T, DM>(gf, b, h2i, phi, ii, jj, kk, nullptr);
+      s += ld(rhs, (unsigned)cidx(gf, ii, jj, kk)) - mac_L<T, DM>(gf, b, h2i, phi, ii, jj, kk, nullptr);
     }
-    rc[t] = (DM == 3 ? T(0.125) : T(0.25)) * s;
-    if (z) z[t] = T(0);
+    const T r = (DM == 3 ? T(0.125) : T(0.25)) * s;
+    rc[t] = r;
+    z[t] = first ? mac_first<T, DM>(gc, bc, h2ic, r, i, j, k) : T(0);
   }
 };
 
@@ -1154,7 +1329,10 @@ struct DivPlusFn {
   Dec dc;
   T* out2 = nullptr;  // optional second copy
   int sp = 0;         // u in parity-split storage
-  T* z = nullptr;     // optional array zeroed (the MAC solve's initial phi)
+  T* z = nullptr;     // optional: the MAC solve's initial phi, zero or (first) mac_first
+  int first = 0;
+  T* b[3] = {nullptr, nullptr, nullptr};
+  T h2i = T(0);
   HD void operator()(long t) const {
     int i, j, k;
     decode3(t, dc, i, j, k);
@@ -1164,7 +1342,7 @@ struct DivPlusFn {
     const T v = bp ? T(s + T(bp[t])) : s;
     out[t] = v;
     if (out2) out2[t] = v;
-    if (z) z[t] = T(0);
+    if (z) z[t] = first ? mac_first<T, DM>(g, b, h2i, v, i, j, k) : T(0);
   }
 };
 
