@@ -2794,6 +2794,173 @@ static int gmres_any(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool w
 }
 
 // ------------------------------------------------------------------------------------------
+#ifndef LMFHD_HOST_DEBUG
+// stochastic_m_fluxdiv with noise generated on the device, unfiltered: every stress value formed
+// once per tile instead of once per face that reads it (18 Philox blocks and quantiles a cell, now
+// 4 blocks and 9 quantiles, and the tile's halo).  A workgroup covers a 32 x 16 tile of (i, j)
+// positions, of which the inner 30 x 14 are its outputs, and marches over zc planes; each thread
+// forms its position's cell stress (3 values of one block) and edge stresses (2 of one block each),
+// keeps those the next plane needs in registers and passes those its x and y neighbours need
+// through LDS.  Bound by arithmetic: of 315 us at 128^3 (760 with a face per thread and the former
+// quantile) about 130 are the generator, the rest the quantiles.  Differences and sums are StochFn's, in
+// its order.
+struct StochTile {
+  Geo g;
+  NoiseGen ng;
+  const double* eta_cc;
+  const double* eta_ed[3];
+  double var, dxinv, sqrt2, ccfac;
+  int one;  // 1: both components of an edge take word 0 (the symmetric form)
+  int incr;
+  double* out[3];
+  double* outp;  // cell part, zeroed unless incr
+  int tx, ty, zc;
+};
+constexpr int STX = 32, STY = 16;
+// 4 waves per SIMD: two workgroups a CU at 128 VGPRs (few spills) beat one at 179
+template <int DM>
+__global__ void __launch_bounds__(STX * STY, 4) k_stoch_tile(StochTile S) {
+  const Geo& g = S.g;
+  __shared__ double ex[6][STY][STX];
+  const int lx = (int)threadIdx.x & (STX - 1), ly = (int)threadIdx.x / STX;
+  const int bx = (int)blockIdx.x % S.tx, br = (int)blockIdx.x / S.tx;
+  const int by = br % S.ty, bz = br / S.ty;
+  const int i = bx * (STX - 2) + lx - 1, j = by * (STY - 2) + ly - 1;
+  const int nzp = DM == 3 ? g.n[2] + 1 : 1;  // planes of the nodal box
+  const int k0 = bz * S.zc, k1 = imin(k0 + S.zc, nzp);
+  // index of the cell that stands at v in direction d (periodic image, or the last inside a wall)
+  auto cell1 = [&](int v, int d) {
+    const int n = g.n[d];
+    if (v < 0) return g.per[d] ? v + n : 0;
+    if (v >= n) return g.per[d] && v - n < n ? v - n : n - 1;
+    return v;
+  };
+  // node at v: the duplicate of a periodic direction takes node 0; the factor of a wall node
+  auto node1 = [&](int v, int d, double& fac) {
+    const int n = g.n[d];
+    v = v < 0 ? 0 : imin(v, n);
+    if (v == 0 && g.wlo[d]) fac *= g.slo[d] < 0 ? S.sqrt2 : 0.0;
+    else if (v == n && g.whi[d]) fac *= g.shi[d] < 0 ? S.sqrt2 : 0.0;
+    else if (v == n && g.per[d]) v = 0;
+    return v;
+  };
+  const int ci = cell1(i, 0), cj = cell1(j, 1);
+  double fx = 1.0, fy = 1.0;
+  const int ni = node1(i, 0, fx), nj = node1(j, 1, fy);
+  auto cells = [&](int k, double* c) {
+    const long o = cidx(g, ci, cj, DM == 3 ? cell1(k, 2) : 0);
+    S.ng.normals<DM>(o, 0, c);
+    const double s = sqrt(S.eta_cc[o] * 1.0);
+#pragma unroll
+    for (int a = 0; a < DM; ++a) c[a] = (S.var * (S.ccfac * c[a])) * s;
+  };
+  auto edges = [&](int e, int a, int b, int c, double fac, double* v) {  // edge array e at (a, b, c)
+    const long o = eidx(g, e, a, b, c);
+    S.ng.normals<2>(o, 1 + e, v);
+    if (S.one) v[1] = v[0];
+    const double s = sqrt(S.eta_ed[e][o] * 1.0);
+    v[0] = fac * ((S.var * v[0]) * s);
+    v[1] = fac * ((S.var * v[1]) * s);
+  };
+  double cz = 0.0, xz[2] = {0.0, 0.0}, yz[2] = {0.0, 0.0};
+  if (DM == 3) {
+    double c[3];
+    cells(k0 - 1, c);
+    cz = c[DM - 1];
+    double fz = 1.0;
+    const int nk = node1(k0, 2, fz);
+    edges(1, ni, cj, nk, fx * fz, xz);
+    edges(2, ci, nj, nk, fy * fz, yz);
+  }
+  const bool inner = lx > 0 && lx < STX - 1 && ly > 0 && ly < STY - 1;
+  for (int k = k0; k < k1; ++k) {
+    double c[3] = {0.0, 0.0, 0.0}, xy[2] = {0.0, 0.0}, xzn[2] = {0.0, 0.0}, yzn[2] = {0.0, 0.0};
+    cells(k, c);
+    if (DM == 2) {
+      edges(0, ni, nj, 0, fx * fy, xy);
+    } else if (k < g.n[2]) {
+      double fz = 1.0;
+      const int nk = node1(k + 1, 2, fz);
+      edges(0, ni, nj, k, fx * fy, xy);
+      edges(1, ni, cj, nk, fx * fz, xzn);
+      edges(2, ci, nj, nk, fy * fz, yzn);
+    }
+    ex[0][ly][lx] = c[0];
+    ex[1][ly][lx] = c[1];
+    ex[2][ly][lx] = xy[0];
+    ex[3][ly][lx] = xy[1];
+    if (DM == 3) {
+      ex[4][ly][lx] = xz[1];
+      ex[5][ly][lx] = yz[1];
+    }
+    __syncthreads();
+    if (inner) {
+      if (face_in(g, 0, i, j, k)) {
+        double v = 0.0;
+        v += (c[0] - ex[0][ly][lx - 1]) * S.dxinv;
+        v += (ex[2][ly + 1][lx] - xy[0]) * S.dxinv;
+        if (DM == 3) v += (xzn[0] - xz[0]) * S.dxinv;
+        double* o = S.out[0] + fidx(g, 0, i, j, k);
+        if (wall_face(g, 0, i)) {
+          if (!S.incr) *o = 0.0;
+        } else {
+          *o = S.incr ? *o + v : v;
+        }
+      }
+      if (face_in(g, 1, i, j, k)) {
+        double v = 0.0;
+        v += (ex[3][ly][lx + 1] - xy[1]) * S.dxinv;
+        v += (c[1] - ex[1][ly - 1][lx]) * S.dxinv;
+        if (DM == 3) v += (yzn[0] - yz[0]) * S.dxinv;
+        double* o = S.out[1] + fidx(g, 1, i, j, k);
+        if (wall_face(g, 1, j)) {
+          if (!S.incr) *o = 0.0;
+        } else {
+          *o = S.incr ? *o + v : v;
+        }
+      }
+      if (DM == 3 && face_in(g, 2, i, j, k)) {
+        double v = 0.0;
+        v += (ex[4][ly][lx + 1] - xz[1]) * S.dxinv;
+        v += (ex[5][ly + 1][lx] - yz[1]) * S.dxinv;
+        v += (c[2] - cz) * S.dxinv;
+        double* o = S.out[2] + fidx(g, 2, i, j, k);
+        if (wall_face(g, 2, k)) {
+          if (!S.incr) *o = 0.0;
+        } else {
+          *o = S.incr ? *o + v : v;
+        }
+      }
+      if (!S.incr && i < g.n[0] && j < g.n[1] && k < g.n[2]) S.outp[cidx(g, i, j, k)] = 0.0;
+    }
+    __syncthreads();
+    cz = c[2];
+    xz[0] = xzn[0];
+    xz[1] = xzn[1];
+    yz[0] = yzn[0];
+    yz[1] = yzn[1];
+  }
+}
+static void launch_stoch_tile(Ctx& c, StochTile S) {
+  const int nzp = c.dm == 3 ? c.g.n[2] + 1 : 1;
+  S.tx = (c.g.n[0] + 1 + STX - 3) / (STX - 2);
+  S.ty = (c.g.n[1] + 1 + STY - 3) / (STY - 2);
+  // planes per workgroup: a march repeats one plane's work, and 512 workgroups run at a time
+  long best = 0;
+  for (int nch = 1; nch <= std::max(1, nzp / 4); ++nch) {
+    const int zc = (nzp + nch - 1) / nch;
+    const long wg = (long)S.tx * S.ty * ((nzp + zc - 1) / zc), cost = (wg + 511) / 512 * (zc + 1);
+    if (nch > 1 && cost >= best) continue;
+    best = cost;
+    S.zc = zc;
+  }
+  const int nb = S.tx * S.ty * ((nzp + S.zc - 1) / S.zc);
+  if (c.dm == 3) hipLaunchKernelGGL(k_stoch_tile<3>, dim3((unsigned)nb), dim3(STX * STY), 0, c.s, S);
+  else hipLaunchKernelGGL(k_stoch_tile<2>, dim3((unsigned)nb), dim3(STX * STY), 0, c.s, S);
+}
+#endif
+
+// ------------------------------------------------------------------------------------------
 // momentum time steps for one species (density and viscosities constant in time, homogeneous
 // velocity boundaries): advance_timestep_inertial / advance_timestep_overdamped, momentum part
 static void step_bufs(Ctx& c) {
@@ -4356,6 +4523,28 @@ static int stoch_dev(lmfhd_ctx* x, unsigned long long seed, unsigned long long s
   }
   const double dz = dm == 3 ? c.dx : c.d.dz2d;
   const double var = std::sqrt(variance_coef_mom * 2.0 * k_B / (c.dx * c.dx * dz * dt));
+#ifndef LMFHD_HOST_DEBUG
+  if (c.d.filtering_width == 0) {
+    StochTile S;
+    S.g = c.g;
+    S.ng.ph.k0 = seed;
+    S.ng.ph.k1 = NOISE_KEY1;
+    S.ng.stage = stage;
+    S.eta_cc = ecc;
+    for (int e = 0; e < 3; ++e) S.eta_ed[e] = eed[e];
+    S.var = var;
+    S.dxinv = 1.0 / c.dx;
+    S.sqrt2 = std::sqrt(2.0);
+    S.ccfac = stoch_stress_form == 0 ? 1.0 : std::sqrt(2.0);
+    S.one = stoch_stress_form == 0 ? 0 : 1;
+    S.incr = increment ? 1 : 0;
+    for (int a = 0; a < 3; ++a) S.out[a] = f + c.off[a < dm ? a : dm - 1];
+    S.outp = f + c.off[3];
+    launch_stoch_tile(c, S);
+    check_launch();
+    return LMFHD_OK;
+  }
+#endif
   StochFn Fs[3];
   for (int a = 0; a < dm; ++a) {
     StochFn F;
