@@ -31,7 +31,7 @@ struct Rec {
   int kind = 0;                   // 0 flat, 1 cols, 2 rows, 3 blocks
   std::vector<unsigned char> f;   // the functor's bytes
   long n = 0;                     // flat: items; blocks: workgroups
-  int ncols = 0, nz = 0, kc = 0;  // cols
+  int ncols = 0, nz = 0;          // cols
   int nw = 0;                     // rows: waves; blocks: threads of a workgroup
   MultiFn multi = nullptr;
 };
@@ -43,14 +43,13 @@ inline Recorder*& rec_slot() {
   return r;
 }
 template <class F>
-inline void record(int kind, const F& f, MultiFn m, long n, int ncols = 0, int nz = 0, int kc = 0, int nw = 0) {
+inline void record(int kind, const F& f, MultiFn m, long n, int ncols = 0, int nz = 0, int nw = 0) {
   Rec r;
   r.kind = kind;
   r.f.assign(reinterpret_cast<const unsigned char*>(&f), reinterpret_cast<const unsigned char*>(&f) + sizeof(F));
   r.n = n;
   r.ncols = ncols;
   r.nz = nz;
-  r.kc = kc;
   r.nw = nw;
   r.multi = m;
   rec_slot()->recs.push_back(std::move(r));
@@ -85,24 +84,25 @@ inline bool xcd_order() {
   return v == 1;
 }
 
-// Column launcher: F::operator()(col, k0, k1) handles point `col` of an (nx*ny) plane for
-// k in [k0, k1).  Logical block lb covers 256 columns of z-run lb / nbx.  Workgroups are handed
-// to the eight XCDs round-robin (hardware block b runs on XCD b % 8), so hardware block b takes
-// logical block (b % 8) * per + b / 8: each XCD walks a contiguous range of z-runs and the
-// neighbouring rows and planes a stencil re-reads stay in that XCD's L2.
+// Column launcher: F::operator()(col, k) handles point `col` of an (nx*ny) plane on plane k.
+// Logical block lb covers 256 columns of plane lb / nbx.  Workgroups are handed to the eight XCDs
+// round-robin (hardware block b runs on XCD b % 8), so hardware block b takes logical block
+// (b % 8) * per + b / 8: each XCD walks a contiguous range of planes and the neighbouring rows and
+// planes a stencil re-reads stay in that XCD's L2.  One plane per thread: a march over several,
+// reusing the planes it has read, lost more occupancy than it gained (128^3 FP64 stag_applyop 75 us
+// with 1 plane, 78 with 2, 90 with 4, 118 with 8), and its loop alone cost registers (152 against
+// 125 in apply_matrix's kernel).
 constexpr int COL_BS = 256;
 #ifndef LMFHD_HOST_DEBUG
 template <class F>
-__global__ void __launch_bounds__(COL_BS) k_cols(F f, int ncols, int nz, int kc, int nbx, int nblog, int per) {
+__global__ void __launch_bounds__(COL_BS) k_cols(F f, int ncols, int nbx, int nblog, int per) {
   const int b = blockIdx.x;
   const int lb = (b & 7) * per + (b >> 3);
   if (lb >= nblog) return;
   const int bz = lb / nbx, bx = lb - bz * nbx;
   const int col = bx * COL_BS + threadIdx.x;
   if (col >= ncols) return;
-  const int k0 = bz * kc;
-  const int k1 = k0 + kc < nz ? k0 + kc : nz;
-  f(col, k0, k1);
+  f(col, bz);
 }
 #endif
 
@@ -115,17 +115,15 @@ constexpr size_t MAX_KERNARG = 4096;
 template <class F>
 void multi_cols(hipStream_t s, const unsigned char* fs, int nent, const Rec& r);
 template <class F>
-inline void launch_cols(hipStream_t s, int ncols, int nz, int kc, const F& f) {
+inline void launch_cols(hipStream_t s, int ncols, int nz, const F& f) {
   static_assert(sizeof(F) + 32 <= MAX_KERNARG, "functor too large for the kernel-argument segment");
   if (ncols <= 0 || nz <= 0) return;
-  if (kc < 1) kc = 1;
   if (rec_slot()) {
-    record(1, f, &multi_cols<F>, 0, ncols, nz, kc);
+    record(1, f, &multi_cols<F>, 0, ncols, nz);
     return;
   }
   const int nbx = (ncols + COL_BS - 1) / COL_BS;
-  const int nbz = (nz + kc - 1) / kc;
-  const int nblog = nbx * nbz;
+  const int nblog = nbx * nz;
   const int per = (nblog + 7) / 8;
 #ifdef LMFHD_HOST_DEBUG
   (void)s;
@@ -135,12 +133,11 @@ inline void launch_cols(hipStream_t s, int ncols, int nz, int kc, const F& f) {
     for (int tx = 0; tx < COL_BS; ++tx) {
       const int col = bx * COL_BS + tx;
       if (col >= ncols) continue;
-      const int k0 = bz * kc;
-      f(col, k0, k0 + kc < nz ? k0 + kc : nz);
+      f(col, bz);
     }
   }
 #else
-  hipLaunchKernelGGL(k_cols<F>, dim3((unsigned)(8 * per)), dim3(COL_BS), 0, s, f, ncols, nz, kc, nbx, nblog, per);
+  hipLaunchKernelGGL(k_cols<F>, dim3((unsigned)(8 * per)), dim3(COL_BS), 0, s, f, ncols, nbx, nblog, per);
 #endif
 }
 
@@ -169,7 +166,7 @@ inline void launch_rows(hipStream_t s, int nw, const F& f) {
   static_assert(sizeof(F) + 32 <= MAX_KERNARG, "functor too large for the kernel-argument segment");
   if (nw <= 0) return;
   if (rec_slot()) {
-    record(2, f, &multi_rows<F>, 0, 0, 0, 0, nw);
+    record(2, f, &multi_rows<F>, 0, 0, 0, nw);
     return;
   }
   const int nblog = (nw + ROW_WAVES - 1) / ROW_WAVES;
@@ -193,14 +190,13 @@ __global__ void __launch_bounds__(256) k_for_multi(const F* __restrict__ fs, lon
   if (t < n) f(t);
 }
 template <class F>
-__global__ void __launch_bounds__(COL_BS) k_cols_multi(const F* __restrict__ fs, int ncols, int nz, int kc, int nbx) {
+__global__ void __launch_bounds__(COL_BS) k_cols_multi(const F* __restrict__ fs, int ncols, int nbx) {
   const F& f = fs[blockIdx.y];
   const int lb = blockIdx.x;
   const int bz = lb / nbx, bx = lb - bz * nbx;
   const int col = bx * COL_BS + threadIdx.x;
   if (col >= ncols) return;
-  const int k0 = bz * kc;
-  f(col, k0, k0 + kc < nz ? k0 + kc : nz);
+  f(col, bz);
 }
 template <class F>
 __global__ void __launch_bounds__(256) k_rows_multi(const F* __restrict__ fs, int nw) {
@@ -223,7 +219,7 @@ void multi_flat(hipStream_t s, const unsigned char* fs, int nent, const Rec& r) 
 }
 template <class F>
 void multi_cols(hipStream_t s, const unsigned char* fs, int nent, const Rec& r) {
-  const int nbx = (r.ncols + COL_BS - 1) / COL_BS, nbz = (r.nz + r.kc - 1) / r.kc;
+  const int nbx = (r.ncols + COL_BS - 1) / COL_BS, nbz = r.nz;
 #ifdef LMFHD_HOST_DEBUG
   (void)s;
   for (int q = 0; q < nent; ++q)
@@ -232,13 +228,12 @@ void multi_cols(hipStream_t s, const unsigned char* fs, int nent, const Rec& r) 
       for (int tx = 0; tx < COL_BS; ++tx) {
         const int col = bx * COL_BS + tx;
         if (col >= r.ncols) continue;
-        const int k0 = bz * r.kc;
-        reinterpret_cast<const F*>(fs)[q](col, k0, k0 + r.kc < r.nz ? k0 + r.kc : r.nz);
+        reinterpret_cast<const F*>(fs)[q](col, bz);
       }
     }
 #else
   hipLaunchKernelGGL(k_cols_multi<F>, dim3((unsigned)(nbx * nbz), (unsigned)nent), dim3(COL_BS), 0, s,
-                     reinterpret_cast<const F*>(fs), r.ncols, r.nz, r.kc, nbx);
+                     reinterpret_cast<const F*>(fs), r.ncols, nbx);
 #endif
 }
 template <class F>
@@ -284,7 +279,7 @@ inline void launch_blocks(hipStream_t s, int nb, const F& f, int nt = F::BS) {
   static_assert(sizeof(F) + 32 <= MAX_KERNARG, "functor too large for the kernel-argument segment");
   if (nb <= 0) return;
   if (rec_slot()) {
-    record(3, f, &multi_blocks<F>, nb, 0, 0, 0, nt);
+    record(3, f, &multi_blocks<F>, nb, 0, 0, nt);
     return;
   }
 #ifdef LMFHD_HOST_DEBUG

@@ -166,6 +166,8 @@ static const int RED_NV = 16;
 // partial sum of workgroup b for product q: q-major, so that the final reduction's lanes (one
 // per b) read consecutive addresses
 #define PART(b, q) ((long)(q) * RED_BLOCKS + (b))
+constexpr int MEAN_BLOCKS = 2048;  // most workgroups of SumItemsBlk (a multiple of 256)
+constexpr int MEAN_CHUNK = 1024;   // elements of a MeanOutBlk workgroup
 
 #ifndef LMFHD_HOST_DEBUG
 __device__ __forceinline__ double wave_sum(double v) {
@@ -259,6 +261,53 @@ struct RedFinalBlk {
   double* out;
   const double* skip;
   __device__ void block(int) const { red_final_block(part, nb, nv, do_sqrt, out, skip); }
+};
+
+// Each of nb workgroups (a multiple of 256) runs per of F's n items, in XCD-contiguous
+// order, and leaves the sum of what they return in part; MeanOutBlk then takes the sum of all of
+// them over cnt from x, each of its workgroups forming that sum itself, in one order.  The mean of
+// the pressure so costs no sweep and no reduction launch of its own.
+template <class F>
+struct SumItemsBlk {
+  static constexpr int BS = 256;
+  F f;
+  long n, per;
+  int nb;
+  double* part;
+  __device__ void block(int b) const {
+    const int lb = (b & 7) * (nb >> 3) + (b >> 3);
+    const long e0 = (long)lb * per, e1 = e0 + per < n ? e0 + per : n;
+    double s = 0.0;
+    for (long e = e0 + threadIdx.x; e < e1; e += 256) s += f.item(e);
+    __shared__ double sh[4];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) part[lb] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+  }
+};
+struct MeanOutBlk {
+  static constexpr int BS = 256;
+  double* x;
+  long n;
+  double cnt;
+  const double* part;
+  int nb;
+  __device__ void block(int b) const {
+    double s = 0.0;
+    for (int q = threadIdx.x; q < nb; q += 256) s += part[q];
+    __shared__ double sh[4];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    const double m = (((sh[0] + sh[1]) + sh[2]) + sh[3]) / cnt;
+    const long e0 = (long)b * MEAN_CHUNK;
+#pragma unroll
+    for (int q = 0; q < MEAN_CHUNK / 256; ++q) {
+      const long e = e0 + q * 256 + threadIdx.x;
+      if (e < n) x[e] -= m;
+    }
+  }
 };
 
 // max |x| of a float or double array (stag_mg_solver residual norms)
@@ -497,6 +546,32 @@ struct RemoveMeanBlk {
 #endif
 
 #ifdef LMFHD_HOST_DEBUG
+template <class F>
+struct SumItemsBlk {
+  static constexpr int BS = 1;
+  F f;
+  long n, per;
+  int nb;
+  double* part;
+  void block_host(int b) const {
+    double s = 0.0;
+    for (long e = b * per; e < std::min(n, (b + 1) * per); ++e) s += f.item(e);
+    part[b] = s;
+  }
+};
+struct MeanOutBlk {
+  static constexpr int BS = 1;
+  double* x;
+  long n;
+  double cnt;
+  const double* part;
+  int nb;
+  void block_host(int b) const {
+    double s = 0.0;
+    for (int q = 0; q < nb; ++q) s += part[q];
+    for (long e = (long)b * MEAN_CHUNK; e < std::min(n, (long)(b + 1) * MEAN_CHUNK); ++e) x[e] -= s / cnt;
+  }
+};
 // host form of mdot (one "workgroup" forms every sum), recordable like the device form
 struct MdotHostBlk {
   static constexpr int BS = 1;
@@ -776,11 +851,9 @@ static bool has_wall(const Geo& g) {
   return false;
 }
 
-// column launches over the nodal (n+1)-box, one plane per thread: measured on MI355X (128^3
-// FP64 stag_applyop 75 us with runs of 1 plane, 78 with 2, 90 with 4, 118 with 8) the
-// register-heavier marching threads lose more occupancy than the plane reuse gains
+// column launches over the nodal (n+1)-box
 struct ColShape {
-  int ncols, nz, kc;
+  int ncols, nz;
   FastDiv cx;
 };
 static ColShape col_shape(const Geo& g) {
@@ -789,7 +862,6 @@ static ColShape col_shape(const Geo& g) {
   c.ncols = nx * ny;
   c.nz = g.dm == 3 ? g.n[2] + 1 : 1;
   c.cx = make_fastdiv((unsigned)nx);
-  c.kc = 1;
   return c;
 }
 // row mapping (launch_rows) of a level: lanes along x in chunks of 64, the x faces i = n_x as
@@ -827,7 +899,7 @@ static void apply_all_cols(hipStream_t s, const Geo& g, const Coefs<T>& C, T* co
   }
   f.cx = cs.cx;
   f.mode = mode;
-  launch_cols(s, cs.ncols, cs.nz, cs.kc, f);
+  launch_cols(s, cs.ncols, cs.nz, f);
 }
 // sp: phi, rhs, out and alpha in parity-split storage (|visc_type| 1 levels only)
 template <typename T, int VT, int DM>
@@ -1301,7 +1373,7 @@ struct StagMG {
     }
     const ColShape cs = col_shape(c.g);
     F.cx = cs.cx;
-    launch_cols(s, cs.ncols, cs.nz, cs.kc, F);
+    launch_cols(s, cs.ncols, cs.nz, F);
   }
   void resid_restrict(hipStream_t s, int n) {
     dispatch_vd(vt, dm, [&](auto V, auto D) { resid_restrict_vd<decltype(V)::value, decltype(D)::value>(s, n); });
@@ -1993,7 +2065,7 @@ static void apply_matrix(Ctx& c, double* x, double* b, Walls walls) {
       }
       const ColShape cs = col_shape(c.g);
       F.cx = cs.cx;
-      launch_cols(s, cs.ncols, cs.nz, cs.kc, F);
+      launch_cols(s, cs.ncols, cs.nz, F);
     };
     if (walls == Walls::any) go(std::integral_constant<int, 1>{});
     else go(std::integral_constant<int, 0>{});
@@ -2035,12 +2107,9 @@ static void stag_applyop64(Ctx& c, double* phi, double* out, int color) {
 
 // null-space handling at the end of apply_precon (apply_precon.f90:433-458): subtract the
 // mean pressure; with theta = 0 and no no-slip wall also the velocity means
-static void precon_tail(Ctx& c, double* x) {
+static void precon_tail_u(Ctx& c, double* x) {
   hipStream_t s = c.s;
   const int dm = c.dm;
-  double* xp = x + c.off[3];
-  c.R.mdot(xp, nullptr, 0, 1, c.nc, false, c.s_tmp());
-  sub_mean(s, xp, c.s_tmp(), (double)c.nc, c.nc);
   if (c.theta == 0.0) {
     bool no_wall_is_no_slip = true;
     for (int d = 0; d < dm; ++d)
@@ -2054,6 +2123,12 @@ static void precon_tail(Ctx& c, double* x) {
   }
   check_launch();
 }
+static void precon_tail(Ctx& c, double* x) {
+  double* xp = x + c.off[3];
+  c.R.mdot(xp, nullptr, 0, 1, c.nc, false, c.s_tmp());
+  sub_mean(c.s, xp, c.s_tmp(), (double)c.nc, c.nc);
+  precon_tail_u(c, x);
+}
 
 // apply_precon, precon_type 1 (apply_precon.f90:103-195,433-460): b -> x (FP64 vectors)
 template <typename T>
@@ -2061,10 +2136,10 @@ static void precon(Ctx& c, StagMG<T>& mg, MacMG<T>& mac, T* macrhs, const double
   hipStream_t s = c.s;
   const int dm = c.dm;
   auto& l0 = mg.L[0];
-  const ColShape cs = col_shape(c.g);
   const bool first = mg.takes_first_level0();
   dispatch_vd(c.d.visc_type, dm, [&](auto V, auto D) {
     constexpr int VT = decltype(V)::value, DM = decltype(D)::value;
+    const ColShape cs = col_shape(c.g);
     AllFacesFn<EnterFn<T, VT, DM>, DM> F;
     F.g = c.g;
     for (int a = 0; a < 3; ++a) {
@@ -2072,7 +2147,7 @@ static void precon(Ctx& c, StagMG<T>& mg, MacMG<T>& mac, T* macrhs, const double
       F.f[a] = EnterFn<T, VT, DM>{b + c.off[q], l0.rhs[q], l0.phi[q], l0.g, l0.C(), mg.omega, l0.sp, first ? 1 : 0};
     }
     F.cx = cs.cx;
-    launch_cols(s, cs.ncols, cs.nz, cs.kc, F);
+    launch_cols(s, cs.ncols, cs.nz, F);
   });
   mg.solve(s, c.R, first);
   // mac_rhs = D x_u + b_p (kept twice: the MAC solve consumes its copy)
@@ -2098,22 +2173,40 @@ static void precon(Ctx& c, StagMG<T>& mg, MacMG<T>& mac, T* macrhs, const double
     launch(s, c.nc, f);
   }
   mac.solve(s, mac_first ? MacMG<T>::Phi::first : MacMG<T>::Phi::zero);
+  // the result, and the mean pressure taken from it (sum_umac_press, apply_precon.f90:433-437)
+  int nb = 0;
   auto leave = [&](auto D) {
     constexpr int DM = decltype(D)::value;
-    FacesCellFn<PreconFaceFn<T>, PreconCellFn<T>, DM> F;
+    SumItemsBlk<PreconExit<T, DM>> B;
+    PreconExit<T, DM>& F = B.f;
     F.g = c.g;
     for (int a = 0; a < 3; ++a) {
       const int q = a < DM ? a : DM - 1;
-      F.f[a] = PreconFaceFn<T>{c.g, l0.phi[q], mac.L[0].phi, c.alpha64[q], x + c.off[q], 1.0 / c.dx, q, Dec{}, l0.sp};
+      F.phi0[a] = l0.phi[q];
+      F.alpha[a] = c.alpha64[q];
+      F.x[a] = x + c.off[q];
     }
-    F.c = PreconCellFn<T>{macrhs, mac.L[0].phi, c.beta64, c.gamma64, x + c.off[3], c.theta, std::abs(c.d.visc_type)};
-    F.cx = cs.cx;
-    launch_cols(s, cs.ncols, cs.nz, cs.kc, F);
+    F.Phi = mac.L[0].phi;
+    F.mac_rhs = macrhs;
+    F.beta = c.beta64;
+    F.gamma = c.gamma64;
+    F.xp = x + c.off[3];
+    F.dxinv = 1.0 / c.dx;
+    F.theta = c.theta;
+    F.avt = std::abs(c.d.visc_type);
+    F.sp = l0.sp;
+    F.dn = make_dec(c.g.n[0] + 1, c.g.n[1] + 1);
+    B.n = (long)(c.g.n[0] + 1) * (c.g.n[1] + 1) * (dm == 3 ? c.g.n[2] + 1 : 1);
+    B.per = (B.n + 256L * MEAN_BLOCKS - 1) / (256L * MEAN_BLOCKS) * 256;
+    B.nb = nb = (int)(((B.n + B.per - 1) / B.per + 255) / 256 * 256);
+    B.part = c.R.part;
+    launch_blocks(s, nb, B);
   };
   if (dm == 3) leave(std::integral_constant<int, 3>{});
   else leave(std::integral_constant<int, 2>{});
-  // subtract the mean pressure (sum_umac_press, apply_precon.f90:433-437)
-  precon_tail(c, x);
+  launch_blocks(s, (int)((c.nc + MEAN_CHUNK - 1) / MEAN_CHUNK), MeanOutBlk{x + c.off[3], c.nc, (double)c.nc, c.R.part, nb});
+  check_launch();
+  precon_tail_u(c, x);
 }
 
 // visc_schur_complement (apply_precon.f90:538-685): x_p = L_mu^-1 D Minv (0 - A0) Minv G
@@ -2402,7 +2495,7 @@ static void record_precon(Ctx& c) {
 }
 static bool same_shape(const Rec& a, const Rec& b) {
   return a.kind == b.kind && a.multi == b.multi && a.f.size() == b.f.size() && a.n == b.n && a.ncols == b.ncols &&
-         a.nz == b.nz && a.kc == b.kc && a.nw == b.nw;
+         a.nz == b.nz && a.nw == b.nw;
 }
 // one round (B.mu held): replay the recordings of the arrived contexts on the batch stream
 static void batch_run(Batch& B) {

@@ -362,9 +362,9 @@ HD bool face_in(const Geo& g, int a, int i, int j, int k) {
   return i < fext(g, a, 0) && j < fext(g, a, 1) && k < fext(g, a, 2);
 }
 
-// all components at once: L phi (mode 0) or rhs - L phi (mode 1), zero on wall faces.  One
-// thread per (i,j) column of the nodal (n+1)-box marches over a run of k, so every array is
-// streamed once per launch and the k-1/k+1 planes are re-read from cache.
+// all components at once: L phi (mode 0) or rhs - L phi (mode 1), zero on wall faces, one thread
+// per position of the nodal (n+1)-box, so every array is streamed once per launch and the k-1/k+1
+// planes are re-read from cache.
 template <typename T, int VT, int DM>
 struct ApplyAllFn {
   Geo g;
@@ -374,26 +374,24 @@ struct ApplyAllFn {
   T* out[3];
   FastDiv cx;  // divides by nx + 1
   int mode;
-  HD void operator()(int col, int k0, int k1) const {
+  HD void operator()(int col, int k) const {
     const int j = (int)fdiv(cx, (unsigned)col);
     const int i = col - j * (int)cx.d;
-    for (int k = k0; k < k1; ++k) {
-      // every component at the nearest face of its box (loads in bounds), then the stores
-      T v[DM];
-      unsigned o[DM];
+    // every component at the nearest face of its box (loads in bounds), then the stores
+    T v[DM];
+    unsigned o[DM];
 #pragma unroll
-      for (int a = 0; a < DM; ++a) {
-        const int ic = imin(i, fext(g, a, 0) - 1), jc = imin(j, fext(g, a, 1) - 1), kc = imin(k, fext(g, a, 2) - 1);
-        const int I[3] = {ic, jc, kc};
-        o[a] = (unsigned)fidx(g, a, ic, jc, kc);
-        const T r = mode == 0 ? T(0) : ld(rhs[a], o[a]);
-        const T L = lphi<T, VT, DM>(g, C, phi, a, ic, jc, kc, nullptr);
-        v[a] = wall_face(g, a, I[a]) ? T(0) : (mode == 0 ? L : r - L);
-      }
-#pragma unroll
-      for (int a = 0; a < DM; ++a)
-        if (face_in(g, a, i, j, k)) st(out[a], o[a], v[a]);
+    for (int a = 0; a < DM; ++a) {
+      const int ic = imin(i, fext(g, a, 0) - 1), jc = imin(j, fext(g, a, 1) - 1), kc = imin(k, fext(g, a, 2) - 1);
+      const int I[3] = {ic, jc, kc};
+      o[a] = (unsigned)fidx(g, a, ic, jc, kc);
+      const T r = mode == 0 ? T(0) : ld(rhs[a], o[a]);
+      const T L = lphi<T, VT, DM>(g, C, phi, a, ic, jc, kc, nullptr);
+      v[a] = wall_face(g, a, I[a]) ? T(0) : (mode == 0 ? L : r - L);
     }
+#pragma unroll
+    for (int a = 0; a < DM; ++a)
+      if (face_in(g, a, i, j, k)) st(out[a], o[a], v[a]);
   }
 };
 
@@ -965,46 +963,26 @@ struct AllFacesFn {
   // every component is evaluated (at the nearest face of its box where (i,j,k) lies outside
   // it, so that all loads stay in bounds) before any result is stored: the stores cannot then
   // hold back the next component's loads
-  HD void operator()(int col, int k0, int k1) const {
+  HD void operator()(int col, int k) const {
     const int j = (int)fdiv(cx, (unsigned)col);
     const int i = col - j * (int)cx.d;
-    for (int k = k0; k < k1; ++k) {
-      typename F::value_type v[DM];
-      int o[DM];
+    typename F::value_type v[DM];
+    int o[DM];
 #pragma unroll
-      for (int a = 0; a < DM; ++a) {
-        const int ic = imin(i, fext(g, a, 0) - 1), jc = imin(j, fext(g, a, 1) - 1), kc = imin(k, fext(g, a, 2) - 1);
-        o[a] = fidx(g, a, ic, jc, kc);
-        v[a] = f[a].eval(ic, jc, kc, o[a], a);
-      }
-#pragma unroll
-      for (int a = 0; a < DM; ++a)
-        if (face_in(g, a, i, j, k)) f[a].put(i, j, k, o[a], a, v[a]);
+    for (int a = 0; a < DM; ++a) {
+      const int ic = imin(i, fext(g, a, 0) - 1), jc = imin(j, fext(g, a, 1) - 1), kc = imin(k, fext(g, a, 2) - 1);
+      o[a] = fidx(g, a, ic, jc, kc);
+      v[a] = f[a].eval(ic, jc, kc, o[a], a);
     }
-  }
-};
-
-// a per-face functor on every component and a per-cell functor, one column launch
-template <class FF, class FC, int DM>
-struct FacesCellFn {
-  Geo g;
-  FF f[3];
-  FC c;
-  FastDiv cx;
-  HD void operator()(int col, int k0, int k1) const {
-    const int j = (int)fdiv(cx, (unsigned)col);
-    const int i = col - j * (int)cx.d;
-    for (int k = k0; k < k1; ++k) {
 #pragma unroll
-      for (int a = 0; a < DM; ++a)
-        if (face_in(g, a, i, j, k)) f[a].at(i, j, k, fidx(g, a, i, j, k));
-      if (i < g.n[0] && j < g.n[1] && k < g.n[2]) c.at(i, j, k, cidx(g, i, j, k));
-    }
+    for (int a = 0; a < DM; ++a)
+      if (face_in(g, a, i, j, k)) f[a].put(i, j, k, o[a], a, v[a]);
   }
 };
 
 // multigrid entry of component a: rhs = b (converted), phi = 0 or (first) stag_first; with sp the
-// level's arrays are in parity-split storage of geometry g
+// level's arrays are in parity-split storage of geometry g.  (Two positions a thread, so that whole
+// lines of both halves are written: 48 us at 128^3 in FP32 against 45.)
 template <typename T, int VT, int DM>
 struct EnterFn {
   struct value_type {
@@ -1346,6 +1324,53 @@ struct DivPlusFn {
   }
 };
 
+// The preconditioner's result: x_u = phi0 - (1/alpha) G Phi on the faces (subtract_weighted_gradp,
+// macproject.f90:318-362), x_p = -chi mac_rhs + theta Phi on the cells (PreconCellFn's chi), one
+// position of the nodal box an item; returns its cell's x_p.
+template <typename T, int DM>
+struct PreconExit {
+  Geo g;
+  const T* phi0[3];     // multigrid solution, in parity-split storage with sp
+  const T* Phi;         // MAC potential
+  const T* mac_rhs;
+  const double* alpha[3];
+  const double* beta;
+  const double* gamma;
+  double* x[3];
+  double* xp;
+  double dxinv, theta;
+  int avt, sp;
+  Dec dn;  // decoder of the nodal box: n_x + 1, n_y + 1
+  HD double item(long t) const {
+    int i, j, k;
+    decode3(t, dn, i, j, k);
+    double v[DM];
+    unsigned o[DM];
+#pragma unroll
+    for (int a = 0; a < DM; ++a) {
+      const int ic = imin(i, fext(g, a, 0) - 1), jc = imin(j, fext(g, a, 1) - 1), kc = imin(k, fext(g, a, 2) - 1);
+      const int I[3] = {ic, jc, kc};
+      o[a] = (unsigned)fidx(g, a, ic, jc, kc);
+      const double gp = ((double)cc_at(Phi, g, ic, jc, kc) -
+                         (double)cc_at(Phi, g, ic - (a == 0), jc - (a == 1), kc - (a == 2))) * dxinv;
+      const double u = (double)ld(phi0[a], lidx(g, a, ic, jc, kc, sp)) - gp * (1.0 / ld(alpha[a], o[a]));
+      v[a] = wall_face(g, a, I[a]) ? 0.0 : u;
+    }
+    const unsigned oc = (unsigned)cidx(g, imin(i, g.n[0] - 1), imin(j, g.n[1] - 1), imin(k, g.n[2] - 1));
+    double w = -(double)ld(mac_rhs, oc);
+    if (avt == 1) w = w * ld(beta, oc);
+    else if (avt == 2) w = w * ld(beta, oc) * 2.0;
+    else { const double tt = w * ld(gamma, oc); w = w * ld(beta, oc) * (4.0 / 3.0) + tt; }
+    w = w + (double)ld(Phi, oc) * theta;
+#pragma unroll
+    for (int a = 0; a < DM; ++a)
+      if (face_in(g, a, i, j, k)) st(x[a], o[a], v[a]);
+    if (i >= g.n[0] || j >= g.n[1] || k >= g.n[2]) return 0.0;
+    st(xp, oc, w);
+    return w;
+  }
+};
+
 // x_u = phi0 - (1/alpha) G Phi (subtract_weighted_gradp, macproject.f90:318-362), FP64 output
 template <typename T>
 struct PreconFaceFn {
@@ -1473,37 +1498,35 @@ struct AmPosFn {
   double* outp;
   double dxinv;
   FastDiv cx;  // divides by nx + 1
-  HD void operator()(int col, int k0, int k1) const {
+  HD void operator()(int col, int k) const {
     const int j = (int)fdiv(cx, (unsigned)col);
     const int i = col - j * (int)cx.d;
-    for (int k = k0; k < k1; ++k) {
-      double v[DM], hi[DM], lo[DM];
-      unsigned o[DM];
-      const int pi = imin(i, g.n[0] - 1), pj = imin(j, g.n[1] - 1), pk = imin(k, g.n[2] - 1);
+    double v[DM], hi[DM], lo[DM];
+    unsigned o[DM];
+    const int pi = imin(i, g.n[0] - 1), pj = imin(j, g.n[1] - 1), pk = imin(k, g.n[2] - 1);
 #pragma unroll
-      for (int a = 0; a < DM; ++a) {
-        const int ic = imin(i, fext(g, a, 0) - 1), jc = imin(j, fext(g, a, 1) - 1), kc = imin(k, fext(g, a, 2) - 1);
-        const int I[3] = {ic, jc, kc};
-        o[a] = (unsigned)fidx(g, a, ic, jc, kc);
-        const GlobalAcc<double, 3, MK> A{xu[a], nullptr, &g, a, 0};
-        const double L = lphi_acc<double, VT, DM>(g, C, xu, a, ic, jc, kc, nullptr, A);
-        const double gp = (cc_at(xp, g, ic, jc, kc) - cc_at(xp, g, ic - (a == 0), jc - (a == 1), kc - (a == 2))) * dxinv;
-        v[a] = wall_face(g, a, I[a]) ? 0.0 : L + gp;
-        const int P[3] = {pi, pj, pk};
-        lo[a] = ld(xu[a], (unsigned)fidx(g, a, pi, pj, pk));
-        hi[a] = ld(xu[a], (unsigned)fidx(g, a, pi + (a == 0), pj + (a == 1), pk + (a == 2)));
-        if (MK) {
-          lo[a] = wall_face(g, a, P[a]) ? 0.0 : lo[a];
-          hi[a] = wall_face(g, a, P[a] + 1) ? 0.0 : hi[a];
-        }
+    for (int a = 0; a < DM; ++a) {
+      const int ic = imin(i, fext(g, a, 0) - 1), jc = imin(j, fext(g, a, 1) - 1), kc = imin(k, fext(g, a, 2) - 1);
+      const int I[3] = {ic, jc, kc};
+      o[a] = (unsigned)fidx(g, a, ic, jc, kc);
+      const GlobalAcc<double, 3, MK> A{xu[a], nullptr, &g, a, 0};
+      const double L = lphi_acc<double, VT, DM>(g, C, xu, a, ic, jc, kc, nullptr, A);
+      const double gp = (cc_at(xp, g, ic, jc, kc) - cc_at(xp, g, ic - (a == 0), jc - (a == 1), kc - (a == 2))) * dxinv;
+      v[a] = wall_face(g, a, I[a]) ? 0.0 : L + gp;
+      const int P[3] = {pi, pj, pk};
+      lo[a] = ld(xu[a], (unsigned)fidx(g, a, pi, pj, pk));
+      hi[a] = ld(xu[a], (unsigned)fidx(g, a, pi + (a == 0), pj + (a == 1), pk + (a == 2)));
+      if (MK) {
+        lo[a] = wall_face(g, a, P[a]) ? 0.0 : lo[a];
+        hi[a] = wall_face(g, a, P[a] + 1) ? 0.0 : hi[a];
       }
-      double s = (hi[0] - lo[0]) * dxinv + (hi[1] - lo[1]) * dxinv;
-      if (DM == 3) s += (hi[DM - 1] - lo[DM - 1]) * dxinv;
-#pragma unroll
-      for (int a = 0; a < DM; ++a)
-        if (face_in(g, a, i, j, k)) st(out[a], o[a], v[a]);
-      if (i < g.n[0] && j < g.n[1] && k < g.n[2]) st(outp, (unsigned)cidx(g, i, j, k), -s);
     }
+    double s = (hi[0] - lo[0]) * dxinv + (hi[1] - lo[1]) * dxinv;
+    if (DM == 3) s += (hi[DM - 1] - lo[DM - 1]) * dxinv;
+#pragma unroll
+    for (int a = 0; a < DM; ++a)
+      if (face_in(g, a, i, j, k)) st(out[a], o[a], v[a]);
+    if (i < g.n[0] && j < g.n[1] && k < g.n[2]) st(outp, (unsigned)cidx(g, i, j, k), -s);
   }
 };
 
