@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from lowmachfhd_amd.grid import NO_SLIP_WALL, PERIODIC, SLIP_WALL, Grid
-from test_gpu_parity import _solver_mod, pair, rel
+from test_gpu_parity import _solver_mod, consistent_u, pair, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -21,6 +21,7 @@ GRIDS = {
     "all_walls": lambda: Grid((16, 24, 12), 1 / 24, bc_lo=(W, W, Q), bc_hi=(W, Q, W)),
     "most_tiles": lambda: Grid((32, 32, 32), 1 / 32),
     "one_too_many": lambda: Grid((32, 32, 34), 1 / 32, bc_lo=(P, P, W), bc_hi=(P, P, W)),
+    "odd_below": lambda: Grid((20, 12, 14), 1 / 20, bc_lo=(P, W, P), bc_hi=(P, W, P)),
     "2d": lambda: Grid((120, 60), 1 / 120),
     "2d_walls": lambda: Grid((72, 100), 1 / 72, bc_lo=(P, W), bc_hi=(P, Q)),
 }
@@ -52,3 +53,32 @@ def test_mac_tiles(gname, cycles):
     finally:
         for kn, d in zip(forms, default):
             S.set_tune(g, {k: d[k] for k in small}, visc_type=-1, **kn)
+
+
+@pytest.mark.parametrize("gname", list(GRIDS))
+@pytest.mark.parametrize("vt", [-1, 1])
+@pytest.mark.parametrize("cycles", [1, 2])
+def test_stag_tiles(gname, vt, cycles):
+    S = _solver_mod()
+    g = GRIDS[gname]()
+    rng = np.random.default_rng(32)
+    small = {"coarse_n": 4, "mac_coarse_n": 4}
+    forms = (dict(precision=S.FP64, krylov=S.GMRES_LEFT), dict(precision=S.MIXED, krylov=S.FGMRES))
+    default = [S.get_tune(g, visc_type=vt, **kn) for kn in forms]
+    more = dict(stag_mg_max_vcycles=cycles, stag_mg_rel_tol=0.0)
+    try:
+        for kn in forms:
+            S.set_tune(g, small, visc_type=vt, **kn)
+        o, s = pair(g, vt, 5.0, rng, **more)
+        bu = consistent_u(g, [rng.standard_normal(g.face_shape(a)) for a in range(g.dm)])
+        ref = o.stag_mg_solve(bu)
+        for kn, tol in zip(forms, (1e-12, 2e-5)):
+            if kn["precision"] == S.MIXED:
+                s = S.StokesSolver(g, visc_type=vt, **more, **kn)
+                s.set_coeffs(*o.coeffs)
+            assert s.tune["coarse_n"] == 4
+            assert rel(s.stag_mg_solver(bu), ref) < tol
+            s.close()
+    finally:
+        for kn, d in zip(forms, default):
+            S.set_tune(g, {k: d[k] for k in small}, visc_type=vt, **kn)
