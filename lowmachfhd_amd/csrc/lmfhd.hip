@@ -228,17 +228,7 @@ __device__ void red_final_block(const double* __restrict__ part, int nb, int nv,
   }
 }
 
-template <int NV>
-__global__ void __launch_bounds__(256) k_mdot(const double* __restrict__ w, const double* __restrict__ V, long vstride,
-                                              int nv, VecLayout L, long n, int weighted, long e0,
-                                              double* __restrict__ part, const double* __restrict__ skip) {
-  mdot_block<NV>((int)blockIdx.x, (int)gridDim.x, w, V, vstride, nv, L, n, weighted, e0, part, skip);
-}
-__global__ void __launch_bounds__(256) k_red_final(const double* __restrict__ part, int nb, int nv, int do_sqrt,
-                                                   double* __restrict__ out, const double* __restrict__ skip) {
-  red_final_block(part, nb, nv, do_sqrt, out, skip);
-}
-// the same two steps as workgroup functors (launch_blocks: recordable)
+// the two steps as workgroup functors (launch_blocks: recordable)
 template <int NV>
 struct MdotBlk {
   static constexpr int BS = 256;
@@ -616,7 +606,7 @@ struct Reducer {
   // skip (device scalar, may be null): when nonzero the products are not formed and out = 0
   void mdot(const double* w, const double* V, long vstride, int nv, long n, bool weighted, double* out_dev,
             bool do_sqrt = false, long e0 = 0, const double* skip = nullptr) {
-    if (nv < 1 || nv > RED_NV) {  // k_mdot reads vector min(q, nv - 1)
+    if (nv < 1 || nv > RED_NV) {  // mdot_block reads vector min(q, nv - 1)
       set_err("internal: mdot over %d vectors", nv);
       throw Fail{LMFHD_E_ARG};
     }
