@@ -182,7 +182,12 @@ struct MacTileBlk {
 // values of their own (odd coarser levels and callers can give them different ones): 0 and n both read
 // n - 1 and 1, n - 1 reads n, 1 reads 0.  Along the component's direction a region is therefore a
 // stretch of the sequence .. n - 1, n, 0, 1, .. with the period n + 1, in which n's neighbour and 0's
-// lie two places on; such a place costs the region a layer more than the other directions.
+// lie two places on.  A face can be swept as often as it has places on its way to the layer loaded
+// around the region, less one for each n | 0 on that way; a face n whose way is one place (the
+// region's last) cannot be swept at all, since the layer holds 0 and not the 1 it reads.  The stored
+// part leaves S places on each side along the component's direction, S - 1 along the others (M): of
+// the S + 1 places to the layer at most one n | 0 is among them (S <= 4, n + 1 >= 5), so every stored
+// face gets its S steps, and what it reads its steps before them.
 // The thin side of the region lies along z, for z faces along y; the pairs lie along x, for x faces
 // along y (a pair's faces differ in parity, which n and 0 do not).
 template <int DM, int A>
@@ -194,7 +199,7 @@ struct StagBox {
   static constexpr int PX = A == 0 ? 1 : 2, PY = A == 0 ? 2 : 1;  // faces of a pair along x, y
   HD static constexpr int R(int d) { return d == 0 ? RX : (d == 1 ? RY : RZ); }
   HD static constexpr int E(int d) { return d == 0 ? 1 : (d == 1 ? LX : LXY); }
-  // layers not stored after S half sweeps
+  // places at either side not stored after S half sweeps (above)
   HD static constexpr int M(int d, int S) { return d >= DM ? 0 : S - 1 + (d == A); }
 };
 // tiles of component a's faces for S half sweeps (extents of at least 4: a period holds the layers)
@@ -212,7 +217,7 @@ template <typename T>
 struct StagPair {  // a thread's faces, [c] of parity c
   T w[2][6], r[2], dg[2];  // weights of the neighbours (VT = -1): normal +, -, transverse +, -, ...
   unsigned o[2];
-  int l[2], m[2];  // in LDS; layers to the nearest side of the region, -1: not there or a wall face
+  int l[2], m[2];  // in LDS; the last half sweep that may take it (from 0), -1: none, or a wall face
   int fix[2];      // bits 0 .. 3: that transverse neighbour is the face's own reflection; 4, 5: the normal
                    // neighbour +, - lies two places on; 6: stored
 };
@@ -289,11 +294,11 @@ struct StagTileBlk {
 #pragma unroll
       for (int d = 0; d < DM; ++d) {
         int lo = U[d], hi = B::R(d) - 1 - U[d];
-        if (d == A && g.per[d]) {  // each n | 0 on the way saves a step
+        if (d == A && g.per[d]) {  // each n | 0 on the way to the loaded layer saves a step
           int c0 = 0, c1 = 0;
           bool z = true;
-          wrap<A>(d, o[d], z, &c0);
-          wrap<A>(d, o[d] + B::R(d) - 1, z, &c1);
+          wrap<A>(d, o[d] - 1, z, &c0);
+          wrap<A>(d, o[d] + B::R(d), z, &c1);
           lo -= cr - c0;
           hi -= c1 - cr;
           fix |= (I[d] == g.n[d] ? 16 : 0) | (I[d] == 0 ? 32 : 0);
