@@ -1860,7 +1860,9 @@ HD bool lsq_norm_hd(const LsqDev& G, int i, const double* prod, const double* sk
   return !lost;
 }
 // least_squares (gmres.f90:531-566) for column i: H(1..i, i) = h1 + h2 (the two Gram-Schmidt
-// passes), H(i+1, i) = |w|; earlier rotations, the new rotation, s, the estimate and the test
+// passes), H(i+1, i) = |w|; earlier rotations, the new rotation, s, the estimate and the test.
+// The column is complete then: a repair that was asked for is done (and steps past the fused
+// sweeps, which end here, must not find an earlier step's request)
 HD void lsq_column_hd(const LsqDev& G, int i, const double* h1, const double* h2, const double* nrm) {
   for (int r = 1; r <= i; ++r) G.h(r, i) = h1[r - 1] + h2[r - 1];
   G.h(i + 1, i) = nrm[0];
@@ -1879,6 +1881,7 @@ HD void lsq_column_hd(const LsqDev& G, int i, const double* h1, const double* h2
   G.stat[0] = est;
   G.stat[1] = (est <= G.thr[0] || est <= G.thr[1]) ? 1.0 : 0.0;
   G.stat[2] = nrm[0];
+  G.stat[3] = 0.0;
 }
 HD void lsq_init_hd(const LsqDev& G, const double* nrm, double thr_rel, double thr_abs) {
   G.sv[1] = nrm[0];
