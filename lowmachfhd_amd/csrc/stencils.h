@@ -1701,8 +1701,12 @@ HD double normal_quantile(double p) {
 struct NoiseGen {
   Philox ph;
   unsigned long long stage;
+  // The uniform number is a double: in the upper half (m + 1/2) 2^-53 rounds to a multiple of 2^-53,
+  // and the last word's, 1 - 2^-54, halfway between its neighbours, to 1, which has no quantile.
+  // That one takes the neighbour below.
   HD static double of_word(unsigned long long w) {
-    return normal_quantile(((double)(w >> 11) + 0.5) * 1.1102230246251565404e-16);
+    const double p = ((double)(w >> 11) + 0.5) * 1.1102230246251565404e-16;
+    return normal_quantile(fmin(p, 1.0 - 1.1102230246251565404e-16));
   }
   // the first N words of the block at (pos, array)
   template <int N>
