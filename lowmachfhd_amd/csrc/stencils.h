@@ -1673,7 +1673,9 @@ HD double normal_quantile(double p) {
                            4.2313330701600911252e1, 1.0);
     return q * n / d;
   }
-  r = sqrt(-log(q < 0.0 ? p : 1.0 - p));
+  // the smaller tail.  p is a double: in the upper half a word's (m + 1/2) 2^-53 has rounded to a
+  // multiple of 2^-53, the last word's 1 - 2^-54 to 1, whose tail is 2^-54 and not 0
+  r = sqrt(-log(fmax(fmin(p, 1.0 - p), 5.5511151231257827021e-17)));
   double x;
   if (r <= 5.0) {
     r -= 1.6;
@@ -1701,12 +1703,8 @@ HD double normal_quantile(double p) {
 struct NoiseGen {
   Philox ph;
   unsigned long long stage;
-  // The uniform number is a double: in the upper half (m + 1/2) 2^-53 rounds to a multiple of 2^-53,
-  // and the last word's, 1 - 2^-54, halfway between its neighbours, to 1, which has no quantile.
-  // That one takes the neighbour below.
   HD static double of_word(unsigned long long w) {
-    const double p = ((double)(w >> 11) + 0.5) * 1.1102230246251565404e-16;
-    return normal_quantile(fmin(p, 1.0 - 1.1102230246251565404e-16));
+    return normal_quantile(((double)(w >> 11) + 0.5) * 1.1102230246251565404e-16);
   }
   // the first N words of the block at (pos, array)
   template <int N>
