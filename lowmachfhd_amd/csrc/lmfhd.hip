@@ -1818,7 +1818,7 @@ struct MacMG {
 // gmres.f90:531-619).  A restart cycle's Givens state lives in device memory -- H, (m+2) x (m+1)
 // and 1-based as in the reference, the rotations cs, sn, the rotated right-hand side s and the
 // solution y -- and one thread does the O(i) work of a column.  The host reads only the status
-// {|s(i+1)|, stop flag, H(i+1, i)} of each step.
+// {|s(i+1)|, stop flag, H(i+1, i), repair flag} of each step.
 struct LsqDev {
   double* H;
   double* cs;
@@ -2221,7 +2221,7 @@ static void precon(Ctx& c, StagMG<T>& mg, MacMG<T>& mac, T* macrhs, const double
     launch_cols(s, cs.ncols, cs.nz, F);
   });
   mg.solve(s, c.R, first);
-  // mac_rhs = D x_u + b_p (kept twice: the MAC solve consumes its copy)
+  // mac_rhs = D x_u + b_p (kept twice: a MAC solve of one level removes its copy's mean)
   const int mac_first = mac.takes_first_level0();
   const T* ph[3] = {l0.phi[0], l0.phi[1], dm == 3 ? l0.phi[2] : l0.phi[1]};
   if (dm == 3) {
@@ -2772,7 +2772,7 @@ static void arnoldi(Ctx& c, double* w, int i) {
   scale_div(s, c.V + (long)i * c.vs, w, nrm, c.vlen);
   lsq_column(c, i);
 }
-// the end of an Arnoldi step whose w' the second pass reduced by more than half of |w'|^2: the
+// the end of an Arnoldi step whose w' the second pass leaves less than half of its norm: the
 // update applied, the norm formed, then the Givens column (the step's stat[3] asks for it)
 static void gs_repair(Ctx& c, double* w, int i) {
   maxpy(c.s, w, c.V, c.vs, i, c.s_h2(), -1.0, c.vlen);
@@ -2965,7 +2965,7 @@ static int gmres_any(Ctx& c, const double* b, double* x, lmfhd_stats* st, bool w
 // positions, of which the inner 30 x 14 are its outputs, and marches over zc planes; each thread
 // forms its position's cell stress (3 values of one block) and edge stresses (2 of one block each),
 // keeps those the next plane needs in registers and passes those its x and y neighbours need
-// through LDS.  Bound by arithmetic: of 315 us at 128^3 (760 with a face per thread and the former
+// through LDS.  Bound by arithmetic: of 313 us at 128^3 (760 with a face per thread and the former
 // quantile) about 130 are the generator, the rest the quantiles.  Differences and sums are StochFn's, in
 // its order.
 struct StochTile {

@@ -1619,8 +1619,9 @@ struct NegDivFn {
 // On-device noise: a counter-based generator, so that every noise value is a pure function of
 // (seed, array, position, stage) and kernels can regenerate it where they need it instead of
 // reading a stored array.  Philox4x64-10 (Salmon, Moraes, Dror & Shaw, SC'11, "Parallel random
-// numbers: as easy as 1, 2, 3"), the uniform ((w >> 11) + 1/2) 2^-53 in (0,1), and the normal
-// quantile, accurate to a few ulp.
+// numbers: as easy as 1, 2, 3"), the uniform ((w >> 11) + 1/2) 2^-53 as a double, and its normal
+// quantile, accurate to a few ulp.  (In the upper half that double is a multiple of 2^-53: beside 1
+// its rounding moves the quantile by far more, 2e-12 of its value where 1 - p is 1e-6.)
 struct Philox {
   unsigned long long k0, k1;
   // the 128-bit product a m: four 32 x 32 + 64 multiply-adds for both halves together
@@ -1654,7 +1655,8 @@ struct Philox {
 // rational function of degree 7 in the centre, |p - 1/2| <= 0.425, and one (beyond p of about
 // 1e-11 another) of sqrt(-log p) in the tails; relative error about 1e-16 before rounding.  No error
 // function and no refinement step: about half the instructions of a rational start with a
-// Halley step on erfc, and 85 % of the lanes need neither logarithm nor root.
+// Halley step on erfc.  85 % of the values lie in the centre, but a wave of 64 has one in the tails in
+// practically every call, so it runs the tail's logarithm and root too.
 // a r^7 + b r^6 + ... + h by Horner's rule (the coefficients as literals: from arrays, the choice
 // between the two tails became loads.  In fused multiply-adds each coefficient took a move into the
 // accumulator, and the moves their place in the registers: 365 us for the 128^3 forcing against 347 at that stage)
